@@ -92,7 +92,8 @@ struct lbm_handle {
   float* ffield32 = nullptr;
   bool ffield_built = false;
   uint64_t ffield_version = 0;  // fields_version the force field was built from
-  // alpha modes 1 and 2: count and list of the cells the correction defers
+  // counters and list of the cells an entropic step's first launch leaves to
+  // its second
   unsigned* defer_count = nullptr;
   int* defer_list = nullptr;
   // datasets of the field file besides density and velocity
@@ -285,6 +286,54 @@ void release(lbm_handle* h) {
   if (h->own_stream && h->stream) (void)hipStreamDestroy(h->stream);
 }
 
+// The smallest domains whose Newton modes take the two-launch solve (power sums,
+// then the listed cells term by term) instead of one term-by-term launch: the
+// latency of two launches against the work of one.  Reference Newton, us a step,
+// one against two: D2Q9 256^2 15 / 25, 384^2 29 / 29, 512^2 36 / 31; D3Q27 32^3
+// 39 / 54, 48^3 100 / 70.
+constexpr int kListMinCells2D = 1 << 18, kListMinCells3D = 1 << 16;
+
+bool certified_mode(const lbm_handle* h) {
+  return h->alpha_mode == LBM_ALPHA_LEARNED || h->alpha_mode == LBM_ALPHA_WARM_RESIDUAL;
+}
+
+// Whether a step lists cells for a second launch (see k_elbm): the certified
+// modes always; on larger domains the Newton modes in 3D and the reference
+// Newton in D2Q9, where the list exists (it is allocated with the handle;
+// without the memory for it the term-by-term kernels solve every cell).  The
+// parity build's reference Newton never does.
+bool newton_lists(const lbm_handle* h) {
+  const bool parity = h->ctype == TYPE_F64 && !h->cfg.shifted;
+  if (h->alpha_mode == LBM_ALPHA_NEWTON && parity) return false;
+  return h->D == 3 ? h->N >= kListMinCells3D
+                   : h->alpha_mode == LBM_ALPHA_NEWTON && h->N >= kListMinCells2D;
+}
+bool lists_cells(const lbm_handle* h) {
+  if (h->cfg.collision != LBM_ELBM || !h->defer_list) return false;
+  return certified_mode(h) || newton_lists(h);
+}
+
+// Shards of the list and cells that one can hold: a workgroup of the first
+// launch lists at most the cells of one row that it covers.
+int list_shards(const lbm_handle* h) {
+  return std::min(h->rows * h->tiles_per_row, kDeferShards);
+}
+int list_capacity(const lbm_handle* h) {
+  const int shards = list_shards(h), blocks = h->rows * h->tiles_per_row;
+  return (blocks + shards - 1) / shards * std::min(h->block, h->nk);
+}
+
+// Two sets of counters, for alternate steps, and the list.
+hipError_t allocate_list(lbm_handle* h) {
+  if (h->defer_list) return hipSuccess;
+  hipError_t e = hipSuccess;
+  if (!h->defer_count) e = hipMalloc(&h->defer_count, 2 * kDeferCounters * sizeof(unsigned));
+  if (e == hipSuccess)
+    e = hipMalloc(&h->defer_list,
+                  (size_t)list_shards(h) * (size_t)list_capacity(h) * sizeof(int));
+  return e;
+}
+
 StepArgs make_args(const lbm_handle* h) {
   StepArgs a{};
   const lbm_config& c = h->cfg;
@@ -309,8 +358,11 @@ StepArgs make_args(const lbm_handle* h) {
   }
   a.alpha_state = h->alpha;
   a.stats = h->stats;
-  a.defer_count = h->defer_count;
-  a.defer_list = h->defer_list;
+  if (lists_cells(h)) {
+    a.defer.cells = h->defer_list;
+    a.defer.shards = list_shards(h);
+    a.defer.capacity = list_capacity(h);
+  }
   a.alpha_mode = h->alpha_mode;
   a.residual_tol = h->residual_tol;
   a.mlp_packed = h->mlp_packed;
@@ -526,6 +578,9 @@ int lbm_create(const lbm_config* cfg, lbm_handle** out) {
       h->err = std::string("alpha field: ") + hipGetErrorString(e);
       return bail(LBM_E_HIP);
     }
+    if (h->N >= (h->D == 3 ? kListMinCells3D : kListMinCells2D) &&
+        allocate_list(h) != hipSuccess)
+      (void)hipGetLastError();  // no room for the list: see lists_cells
   }
   *out = h;
   return LBM_OK;
@@ -843,14 +898,12 @@ int lbm_step(lbm_handle* h, int nsteps, int store_last) {
                 "lbm_mlp_set_normalization");
   if (h->cfg.collision == LBM_ELBM && h->alpha_mode == LBM_ALPHA_LEARNED)
     if (int rc = pack_mlp(h)) return rc;
-  if (h->cfg.collision == LBM_ELBM &&
-      (h->alpha_mode == LBM_ALPHA_LEARNED || h->alpha_mode == LBM_ALPHA_WARM_RESIDUAL)) {
-    // each buffer on its own, so a failed second allocation leaks nothing
-    // when the next call retries
-    if (!h->defer_count) HIP_TRY(h, hipMalloc(&h->defer_count, sizeof(unsigned)));
-    if (!h->defer_list) HIP_TRY(h, hipMalloc(&h->defer_list, (size_t)h->N * sizeof(int)));
-  }
+  if (h->cfg.collision == LBM_ELBM && certified_mode(h)) HIP_TRY(h, allocate_list(h));
   StepArgs a = make_args(h);
+  // +0.0 is the all-zero bit pattern of the counters; a fill kernel, not a
+  // memset, so that the steps can be captured in a graph
+  if (a.defer.cells)
+    HIP_TRY(h, launch_fill(TYPE_F32, h->defer_count, 0.0, 2 * kDeferCounters, h->stream));
   // Vector kernel: one wavefront per 64 V-cell segment, kVecWaves per workgroup.
   const int grid = h->vec ? (h->rows * h->tiles_per_row + kVecWaves - 1) / kVecWaves
                           : h->rows * h->tiles_per_row;
@@ -872,6 +925,10 @@ int lbm_step(lbm_handle* h, int nsteps, int store_last) {
     a.src = h->f[h->cur];
     a.dst = h->f[1 - h->cur];
     a.store = (store_last && s == nsteps - 1) ? 1 : 0;
+    if (a.defer.cells) {
+      a.defer.count = h->defer_count + (s & 1) * kDeferCounters;
+      a.defer.next = h->defer_count + (1 - (s & 1)) * kDeferCounters;
+    }
     a.log_salt = h->log_salt + (unsigned)h->steps * 0x9E3779B9u;
     if (a.store) {
       a.rho_out = h->fields;

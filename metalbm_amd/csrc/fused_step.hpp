@@ -11,6 +11,7 @@
 // operation order (parity build); otherwise the shifted/FMA form is used.
 #pragma once
 
+#include "entropy_series.hpp"
 #include "mlp.hpp"
 #include "step_kernels.hpp"
 
@@ -149,37 +150,42 @@ struct Fp64View {
     asm volatile("" : "+v"(v));
     return double(v);
   }
+  // f - w, and the non-equilibrium part in single precision.
+  template <int i>
+  __device__ __forceinline__ double shifted() const {
+    return SH ? double(fs[i]) : double(fs[i]) - L::W[i];
+  }
+  template <int i>
+  __device__ __forceinline__ float n32() const {
+    return float(ns[i]);
+  }
 };
 
-// ELBM alpha (Collision.h:351-375), first part: the deviation test
-// (Collision.h:284-303) and alphaMax (Collision.h:305-326).  Returns true when
-// the cell needs the root solve; otherwise alpha and branch are final
-// (0: deviation small -> 2; 1: alphaMax < 2 -> 0.95 alphaMax).  p views
-// the pulled populations and their non-equilibrium parts in FP64.  REFDIV
-// keeps the reference's divisions in the deviation test.
-template <class L, bool REFDIV, class V>
-__device__ __forceinline__ bool elbm_prelude(const V& p, double& alpha,
-                                             double& amax, int& branch) {
-  constexpr int Q = L::dimQ;
+// The parity build's deviation test (Collision.h:284-303), with the
+// reference's divisions.
+template <class L, class V>
+__device__ __forceinline__ bool small_deviation_ref(const V& p) {
   bool small = true;
-  static_for<Q>([&](auto ic) {
+  static_for<L::dimQ>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
-    const double fi = p.template f<i>(), ni = p.template n<i>();
-    if constexpr (REFDIV) {
-      const double dev = fabs(ni) / fi;
-      if (dev > 1.0e-3) small = false;
-    } else {
-      if (!(fabs(ni) <= 1.0e-3 * fi) && fi > 0.0) small = false;
-    }
+    const double dev = fabs(p.template n<i>()) / p.template f<i>();
+    if (dev > 1.0e-3) small = false;
   });
-  if (small) {
-    branch = 0;
-    alpha = 2.0;
-    return false;
-  }
+  return small;
+}
+
+// alphaMax (Collision.h:305-326).  True when it is below 2: the cell then
+// takes alpha = 0.95 alphaMax (Collision.h:365-367) and needs no root.
+// REFDIV keeps the reference's divisions; otherwise the smallest ratio is
+// found by cross-multiplied comparisons (num / den < 2.5 tracked as a pair)
+// and one division at the end instead of Q: the products round, so two ratios
+// within an ulp may be ordered either way, which moves alphaMax by at most an
+// ulp.
+template <class L, bool REFDIV, class V>
+__device__ __forceinline__ bool alpha_capped(const V& p, double& alpha, double& amax) {
   amax = 2.5;
   if constexpr (REFDIV) {
-    static_for<Q>([&](auto ic) {
+    static_for<L::dimQ>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
       const double fi = p.template f<i>(), ni = p.template n<i>();
       if (ni > 0) {
@@ -188,14 +194,10 @@ __device__ __forceinline__ bool elbm_prelude(const V& p, double& alpha,
       }
     });
   } else {
-    // The smallest ratio by cross-multiplied comparisons (num / den < 2.5
-    // tracked as a pair) and one division at the end instead of Q: the
-    // products round, so two ratios within an ulp may be ordered either
-    // way, which moves amax by at most an ulp.
     double num = 2.5, den = 1.0;
-    static_for<Q>([&](auto ic) {
+    static_for<L::dimQ>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
-      const double fi = fabs(p.template f<i>()), ni = p.template n<i>();
+      const double fi = fabs(p.template f_fresh<i>()), ni = p.template n_fresh<i>();
       if (ni > 0 && fi * den < num * ni) {
         num = fi;
         den = ni;
@@ -204,47 +206,63 @@ __device__ __forceinline__ bool elbm_prelude(const V& p, double& alpha,
     if (den != 1.0 || num != 2.5) amax = num / den;
   }
   if (amax < 2.) {
-    branch = 1;
     alpha = 0.95 * amax;
-    return false;
+    return true;
   }
-  return true;
+  return false;
 }
 
-// The reference Newton-Raphson (EntropicStep.h:111-140 via solveAlpha,
-// Collision.h:328-349): warm start, |step| <= 1e-8, at most 50 iterations,
-// the iterate before the last step is returned, alpha = 2 when it fails or
-// leaves (1, alphaMax).  G and G' share one log per term.  REFORDER keeps the
-// reference's term order g += f A - fm lg (EntropicStep.h:31-62) with
-// A_i = ln(f_i / w_i) held per term, for FP64 parity; otherwise the constant
-// part is summed once, G = sum f A - sum fm lg, which frees the Q FP64 values
-// of A (the solve's register footprint bounds its occupancy).
-template <class L, bool REFORDER, class V>
-__device__ __forceinline__ double newton_reference(const V& p, double guess,
-                                                   double amax, int& branch,
-                                                   int& iterations) {
+// Newton on the entropy equation term by term, one library logarithm per
+// population and iterate: the whole solve of the parity build, and of the
+// cells beyond the power-sum series (entropy_series.hpp) in the others.
+//  * tol == 0: the reference Newton-Raphson (EntropicStep.h:111-140 via
+//    solveAlpha, Collision.h:328-349): warm start, |step| <= 1e-8, at most 50
+//    iterations, the iterate before the last step is returned, alpha = 2 when
+//    it fails or leaves (1, alphaMax).
+//  * RESIDUAL: the same iteration stopped at |G| <= tol.  Like the reference's
+//    loop it bounds alpha only at convergence: an iterate where a logarithm is
+//    undefined (G is NaN there) or at or below 0 (from where the reference
+//    converges to the trivial root) ends in the fallback alpha = 2.
+// G and G' share one log per term: the library's of f / w in D2Q9 and the
+// parity build, log_or_nan in 3D (27 library logarithms an iterate were most
+// of its solve).  REFORDER keeps the reference's term order
+// g += f A - fm lg (EntropicStep.h:31-62) with A_i = ln(f_i / w_i) held per
+// term, for FP64 parity; otherwise the constant part is summed once, G =
+// sum f A - sum fm lg, and the populations are converted afresh per iteration,
+// so that neither Q FP64 values of A nor 2Q converted doubles are held (the
+// solve's register footprint bounds its occupancy).
+template <class L, bool REFORDER>
+__device__ __forceinline__ double log_term(double v, double w) {
+  if constexpr (REFORDER || L::dimQ <= 9)
+    return log(v / w);
+  else
+    return log_or_nan(v * (1.0 / w));
+}
+template <class L, bool REFORDER, bool RESIDUAL, class V>
+__device__ __forceinline__ double newton_termwise(const V& p, double guess, double amax,
+                                                  double tol, int& branch, int& iterations) {
   constexpr int Q = L::dimQ;
   double A[REFORDER ? Q : 1];
   double SA = 0.0;
   static_for<Q>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
-    const double a = log(p.template f<i>() / L::W[i]);
+    const double fi = REFORDER ? p.template f<i>() : p.template f_fresh<i>();
+    const double a = log_term<L, REFORDER>(fi, L::W[i]);
     if constexpr (REFORDER)
       A[i] = a;
     else
-      SA += p.template f<i>() * a;
+      SA += fi * a;
   });
   double x = guess, step = 0.0;
   bool ok = false;
   iterations = 0;
   for (int it = 1; it <= 50; ++it) {
     x = x - step;
+    if (RESIDUAL && !(x > 0.0)) break;
     iterations = it;
     double g = REFORDER ? 0.0 : SA, dg = 0.0;
     static_for<Q>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
-      // outside the parity build, converted afresh per iteration (no 2Q
-      // doubles held across the loop)
       double fi, ni;
       if constexpr (REFORDER) {
         fi = p.template f<i>();
@@ -254,15 +272,22 @@ __device__ __forceinline__ double newton_reference(const V& p, double guess,
         ni = p.template n_fresh<i>();
       }
       const double fm = fi - x * ni;
-      const double lg = log(fm / L::W[i]);
+      const double lg = log_term<L, REFORDER>(fm, L::W[i]);
       if constexpr (REFORDER)
         g += fi * A[i] - fm * lg;
       else
         g -= fm * lg;
       dg += ni * (1 + lg);
     });
+    // both sums end here: otherwise the compiler moves G' behind the test of G
+    // and holds the Q logarithms until then (235 registers in D3Q27, not 140)
+    if constexpr (RESIDUAL) asm volatile("" : "+v"(g), "+v"(dg));
+    if (RESIDUAL && fabs(g) <= tol) {
+      ok = (x > 1. && x < amax);
+      break;
+    }
     step = g / dg;
-    if (fabs(step) <= 1e-8) {
+    if (!RESIDUAL && fabs(step) <= 1e-8) {
       ok = (x > 1. && x < amax);
       break;
     }
@@ -270,7 +295,7 @@ __device__ __forceinline__ double newton_reference(const V& p, double guess,
     // later iterate NaN, so the reference's loop runs out its 50 iterations
     // and falls back: end now with the same outcome and iteration count.
     // (One such lane would otherwise hold its wavefront for all 50.)
-    if (step != step) {
+    if (!RESIDUAL && step != step) {
       iterations = 50;
       break;
     }
@@ -283,11 +308,79 @@ __device__ __forceinline__ double newton_reference(const V& p, double guess,
   return x;
 }
 
-// Residual solvers (modes 1, 2, 4) evaluate G in the reference's log form
-// for D3Q27 (register budget) and in the log1p-series form for D2Q9 (cheaper
-// where every |alpha x_i| is small).
-template <class L>
-constexpr bool kLogResidual = L::dimQ > 9;
+// newton_termwise for one cell by a group of 32 lanes that all hold it: lane i
+// takes the logarithm of population i, and every lane sums the terms in the
+// same order as newton_termwise, so the results are the same to the bit.  For
+// the short lists of the 3D lattices, whose launch lasts as long as its
+// slowest cell: a solve of 27 logarithms an iterate, up to 50 iterates, took
+// 127 us (D3Q27 256^3) with a lane to a cell and the library's logarithm.  lg: 64 doubles of LDS per
+// wavefront.
+constexpr int kGroupLanes = 32;
+
+template <class L, bool RESIDUAL, class V>
+__device__ __forceinline__ double newton_group(const V& p, double guess, double amax, double tol,
+                                               double* lg, int& branch, int& iterations) {
+  constexpr int Q = L::dimQ;
+  static_assert(Q <= kGroupLanes, "one lane per population");
+  const int lane = threadIdx.x & 63, mine = lane & (kGroupLanes - 1);
+  const double* terms = lg + (lane & ~(kGroupLanes - 1));
+  // lanes beyond Q repeat population 0
+  double fl = p.template f<0>(), nl = p.template n<0>(), iwl = 1.0 / L::W[0];
+  static_for<Q>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    if (mine == i) {
+      fl = p.template f<i>();
+      nl = p.template n<i>();
+      iwl = 1.0 / L::W[i];
+    }
+  });
+  auto share = [&](double v) {
+    wave_sync_lds();  // the previous terms have been read
+    lg[lane] = v;
+    wave_sync_lds();
+  };
+  share(log_or_nan(fl * iwl));
+  double SA = 0.0;
+  static_for<Q>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    SA += p.template f_fresh<i>() * terms[i];
+  });
+  double x = guess, step = 0.0;
+  bool ok = false;
+  iterations = 0;
+  for (int it = 1; it <= 50; ++it) {
+    x = x - step;
+    if (RESIDUAL && !(x > 0.0)) break;
+    iterations = it;
+    share(log_or_nan((fl - x * nl) * iwl));
+    double g = SA, dg = 0.0;
+    static_for<Q>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      const double fi = p.template f_fresh<i>(), ni = p.template n_fresh<i>();
+      const double l = terms[i];
+      g -= (fi - x * ni) * l;
+      dg += ni * (1 + l);
+    });
+    if constexpr (RESIDUAL) asm volatile("" : "+v"(g), "+v"(dg));
+    if (RESIDUAL && fabs(g) <= tol) {
+      ok = (x > 1. && x < amax);
+      break;
+    }
+    step = g / dg;
+    if (!RESIDUAL && fabs(step) <= 1e-8) {
+      ok = (x > 1. && x < amax);
+      break;
+    }
+    // as in newton_termwise; the residual iteration is not a number from here
+    // on either, and ends in the fallback
+    if (step != step) {
+      if (!RESIDUAL) iterations = 50;
+      break;
+    }
+  }
+  branch = ok ? 2 : 3;
+  return ok ? x : 2.0;
+}
 
 __device__ __forceinline__ unsigned sample_hash(unsigned cell, unsigned salt) {
   unsigned h = cell * 0x9E3779B1u ^ salt;
@@ -298,48 +391,51 @@ __device__ __forceinline__ unsigned sample_hash(unsigned cell, unsigned salt) {
   return h ^ (h >> 16);
 }
 
-// Entropic step, one instantiation per alpha solver MODE (0: reference
-// Newton; 1: network start, 2: stored-alpha start, each with a certified
-// correction and plain Newton as fallback; 3: that fallback over the
-// deferred cells; 4: plain Newton from the stored alpha to the residual
-// tolerance for every cell) so that no kernel carries the registers of
-// another's solver.  Plain Newton here is the reference's iteration stopped
-// at |G| <= residual_tol: it falls back to alpha = 2 exactly where the
-// reference Newton does and otherwise reaches the same root.
+// Entropic step, one instantiation per alpha solver MODE so that no kernel
+// carries the registers of another's solver:
+//   6  reference Newton term by term (the parity build; small D2Q9 domains)
+//   0  reference Newton from the power sums; the cells that need the terms are
+//      listed for MODE 5, which solves those
+//   4  plain Newton from the stored alpha to the residual tolerance: 3D from
+//      the power sums, with a list for MODE 7; D2Q9 in the log1p form
+//   1, 2  certified correction of the network's / the stored alpha, else plain
+//      Newton: 3D from the same power sums, with a list for MODE 7; D2Q9 in the
+//      log1p form, with a list for MODE 3.  MODE 1 makes one correction, MODE 2
+//      up to two in 3D: from the stored alpha its iterates are the reference
+//      Newton's own, so whatever it accepts is the root that Newton converges
+//      to; from the network's a second step would also reach roots from which
+//      the reference Newton, started at the stored alpha, diverges to its
+//      alpha = 2 fallback, and the first stands only where that Newton provably
+//      reaches it (reference_reaches)
+// Plain Newton is the reference's iteration stopped at |G| <= residual_tol: it
+// falls back to alpha = 2 exactly where the reference Newton does and otherwise
+// reaches the same root.  A listed cell's populations, alpha and fields are
+// left as they were for the second launch (whose order, set by atomics, enters
+// no result): about 3% of the cells of MODE 0 in D2Q9 2048^2, which cost the
+// whole wavefront the term-by-term solve when they took it in place (468 us a
+// step), and 45 us in dense wavefronts of their own.
+//
+// Measured per step, term by term for every cell -> power sums and list:
+// reference Newton D2Q9 2048^2 474 -> 206 us, D3Q27 256^3 5.75 -> 1.77 ms; plain
+// Newton D3Q27 4.83 -> 1.76 ms, stored-alpha correction D3Q27 4.23 -> 1.78 ms.
+// D2Q9's other modes take one or two evaluations in the log1p form already,
+// most of what the power sums cost (147-167 us of 153), and stay.
 // Three phases so that the learned mode's wavefront-wide matrix-core
 // inference runs with every lane present: (1) pull, moments, fneq and the
-// alpha prelude per cell; (2) MODE 1 only: the network predicts alpha for
+// deviation test per cell; (2) MODE 1 only: the network predicts alpha for
 // every lane's cell at once on the matrix cores; (3) the alpha solve, the
 // collision and the stores per cell.  The workgroup stages the network in
 // LDS once, before phase 1, and one barrier before phase 2 publishes it (a
 // copy per wavefront, as first built, needed four times the LDS and held a
 // D3Q27 workgroup pair at the 160 KiB limit).
-// Minimum wavefronts per SIMD the register allocator must leave room for
-// (the FP64 solve is latency-bound, so occupancy beats a few spills; measured
-// on one MI355X at 2048^2 / 256^3): D2Q9 learned, stored-alpha and plain
-// Newton four (128 VGPRs with 2 and 4 spilled, 109 without: +10%, +12%,
-// +5% over three); D3Q27 learned three (168 VGPRs, none spilled; its launch
-// 3.81 -> 3.47 ms against two); the other D3Q27 solvers two (reference
-// Newton 2.72 k vs 2.03 k MLUPS at one wavefront with 289 registers; at
-// three it spills 42 VGPRs).
-// Workgroups of the MODE 3 launch: eight per CU, enough to keep every SIMD
-// busy at the entropic kernels' occupancy (two to four wavefronts per SIMD)
-// while the list is long.
-constexpr int kDeferBlocks = 2048;
+template <int MODE>
+constexpr bool kListMode = MODE == 3 || MODE == 5 || MODE == 7;
 
-// Resets the deferred-solve counter before the correction launch (a kernel,
-// not a memset, so that the step can be captured in a graph).
-template <int UNUSED = 0>
-__global__ void k_defer_reset(unsigned* count) {
-  if (threadIdx.x == 0) *count = 0u;
-}
-
+// Minimum wavefronts per SIMD the register allocator must leave room for.
 template <class L, int MODE>
 constexpr int elbm_min_waves() {
-  if (L::Type == LatticeType::D2Q9 && (MODE == 1 || MODE == 2 || MODE == 4)) return 4;
-  if (L::Type == LatticeType::D3Q27 && MODE == 1) return 3;
-  if (L::Type == LatticeType::D3Q27) return 2;
-  return 1;
+  if (L::Type == LatticeType::D2Q9) return kListMode<MODE> || MODE == 6 ? 2 : 4;
+  return MODE == 6 ? 2 : 3;
 }
 
 template <class L, class S, class C, int FS, int EQ, bool SH, int BLOCK, int MODE>
@@ -348,6 +444,12 @@ __global__ void __launch_bounds__(BLOCK)
     k_elbm(const StepArgs a, int FSX) {
   constexpr int Q = L::dimQ;
   constexpr bool REF = std::is_same_v<C, double> && !SH;
+  constexpr bool FLAT = L::dimQ <= 9;  // D2Q9
+  // Solves from the power sums.
+  constexpr bool SERIES = MODE == 0 || (!FLAT && (MODE == 1 || MODE == 2 || MODE == 4));
+  // A short list of the 3D Newton modes gives each cell a group of lanes.
+  constexpr bool GROUPS = !FLAT && (MODE == 5 || MODE == 7);
+  __shared__ double s_group[GROUPS ? BLOCK : 1];
   using Shape = MlpShape<L>;
   __shared__ unsigned int s_cnt[6];
   extern __shared__ __align__(16) char s_lds[];
@@ -360,29 +462,41 @@ __global__ void __launch_bounds__(BLOCK)
   char* wave_tile = s_lds + Lay::NET + (threadIdx.x >> 6) * Lay::TILE;
   if constexpr (MODE == 1)
     copy_packed_network<Shape::NIN, Shape::H1, Shape::H2>(a.mlp_packed, s_lds);
-  // MODE 3: plain Newton for the cells the correction of MODE 1 or 2
-  // deferred, one thread per listed cell, the workgroups striding over the
-  // list (a launch of at most kDeferBlocks workgroups: when nothing was
-  // deferred it costs little more than an empty launch).  Every other mode
-  // makes one pass.
-  // With the log-form plain Newton (Q > 9) the striding loop's state cost
-  // 23 spilled registers, so there MODE 3 makes one pass over a full grid
-  // (one thread per possible list entry) instead.
-  constexpr bool STRIDED = MODE == 3 && !kLogResidual<L>;
-  const int n_listed = MODE == 3 ? (int)*a.defer_count : 0;
-  // The striding MODE 3 tallies its statistics per thread over the passes
-  // (branches 0-3, Newton iterations, accepted corrections) and adds them up
-  // once at the end, so that the passes need no barrier.
+  // List modes: a thread or a group of lanes per listed cell, the workgroups
+  // striding over the list.  They tally their statistics per thread over the passes (branches
+  // 0-3, Newton iterations, accepted corrections) and add them up once at the
+  // end, so that the passes need no barrier.  Every other mode makes one pass.
+  constexpr bool LIST = kListMode<MODE>;
+  // The list is kept in shards (see DeferList); each has gridDim.x / shards
+  // workgroups here.
+  int n_listed = a.N, list_block = blockIdx.x, list_blocks = gridDim.x;
+  const int* list = nullptr;
+  if constexpr (LIST) {
+    if (a.defer.cells) {
+      const int shard = blockIdx.x % a.defer.shards;
+      n_listed = (int)a.defer.count[shard * kDeferStride];
+      list = a.defer.cells + (size_t)shard * a.defer.capacity;
+      list_block = blockIdx.x / a.defer.shards;
+      list_blocks = gridDim.x / a.defer.shards;
+      if (list_block == 0 && threadIdx.x == 0) a.defer.next[shard * kDeferStride] = 0u;
+    }
+  }
+  // at most one pass of groups: at 64 cells a shard and more, lanes are few
+  // enough for one each
+  const bool groups = GROUPS && n_listed <= list_blocks * (BLOCK / kGroupLanes);
+  const int group_log2 = groups ? 5 : 0;
+  static_assert(kGroupLanes == 32, "group_log2");
   unsigned tally[6] = {0u, 0u, 0u, 0u, 0u, 0u};
-  for (int list_base = blockIdx.x * BLOCK;; list_base += gridDim.x * BLOCK) {
-  if constexpr (MODE == 3) {
+  for (long long list_base = (long long)list_block * (BLOCK >> group_log2);;
+       list_base += (long long)list_blocks * (BLOCK >> group_log2)) {
+  if constexpr (LIST) {
     if (list_base >= n_listed) break;  // uniform over the workgroup
   }
   CellPos c;
-  if constexpr (MODE == 3) {
-    const int t = list_base + threadIdx.x;
+  if constexpr (LIST) {
+    const long long t = list_base + (threadIdx.x >> group_log2);
     if (t < n_listed) {
-      c = cell_from_index<L>(a, a.defer_list[t]);
+      c = cell_from_index<L>(a, list ? list[t] : (int)t);
     } else {
       c = CellPos{};
       c.active = false;
@@ -396,6 +510,7 @@ __global__ void __launch_bounds__(BLOCK)
   C f[Q], fneq[Q], eqv[Q], F[3];
   C rho = C(1), u[3] = {C(0), C(0), C(0)}, u2 = C(0), drho = C(0);
   double alpha = 2.0, amax = 2.5;
+  CellRange range;
   // Every mode keeps the alpha state (Algorithm.h:103-106): it is the
   // reference Newton's warm start, also when that Newton is the fallback of
   // the residual modes.
@@ -428,8 +543,16 @@ __global__ void __launch_bounds__(BLOCK)
         fneq[i] = f[i] - eqv[i];
       });
     }
-    // The alpha solve runs in FP64 whatever the compute type.
-    solve = elbm_prelude<L, REF>(Fp64View<L, C, SH>{f, fneq}, alpha, amax, branch);
+    // The alpha solve runs in FP64 whatever the compute type.  Branch 0: the
+    // deviation is small and alpha = 2 (Collision.h:356-359).
+    const Fp64View<L, C, SH> p{f, fneq};
+    if constexpr (REF && MODE == 6) {
+      solve = !small_deviation_ref<L>(p);
+    } else {
+      range = cell_range<L>(p);
+      solve = !small_deviation<L>(p, range);
+    }
+    if (!solve) branch = 0;
   }
   // ---- phase 2 ----
   double start = 2.0;
@@ -451,64 +574,88 @@ __global__ void __launch_bounds__(BLOCK)
     C* __restrict__ astate = static_cast<C*>(a.alpha_state);
     if (solve) {
       const Fp64View<L, C, SH> p{f, fneq};
-      if constexpr (MODE == 0) {
-        alpha = newton_reference<L, REF>(p, double(astate[cell]), amax, branch, its);
-      } else if constexpr (MODE == 4 || MODE == 3) {
-        // plain Newton from the stored alpha to the residual tolerance: the
-        // whole solve in MODE 4, the fallback of the cells MODE 1 or 2
-        // deferred in MODE 3
-        if constexpr (kLogResidual<L>) {
-          EvalCurv cv;
-          branch = residual_newton_log<L, false, false>(p, amax, double(astate[cell]),
-                                                        a.residual_tol, 50, alpha, its, cv)
-                       ? 2
-                       : 3;
-          if (branch == 3) alpha = 2.0;
-        } else {
-          alpha = newton_residual<L>(p, amax, double(astate[cell]), a.residual_tol, branch,
-                                     its);
-        }
-      } else {
-        // MODE 1 starts from the network's alpha, MODE 2 from the stored one;
-        // if the solve below is not accepted plain Newton decides -- in the
-        // MODE 3 launch that follows, from the untouched stored alpha, with
-        // the reference's outcome.
-        // MODE 1 makes one certified correction.  MODE 2 (D3Q27) may take a
-        // second: from the stored alpha its iterates are the reference
-        // Newton's own, so whatever it accepts is the root that Newton
-        // converges to.  From the network's alpha a second step would also
-        // reach roots from which the reference Newton, started at the stored
-        // alpha, diverges to its alpha = 2 fallback.
-        if constexpr (MODE == 2) start = double(astate[cell]);
-        int ev = 0;
-        its = ev;
-        bool accepted;
-        EvalCurv cv;
-        if constexpr (kLogResidual<L>)
-          accepted = residual_newton_log<L, true, MODE == 2>(p, amax, start, a.residual_tol,
-                                                             MODE == 1 ? 1 : 2, alpha, ev, cv);
+      const double stored = double(astate[cell]);
+      if constexpr (MODE == 5 || MODE == 6 || MODE == 7) {
+        if (alpha_capped<L, REF && MODE == 6>(p, alpha, amax))
+          branch = 1;
+        else if (groups)
+          alpha = newton_group<L, MODE == 7>(p, stored, amax, a.residual_tol,
+                                             s_group + (GROUPS ? threadIdx.x & ~63 : 0), branch,
+                                             its);
         else
-          accepted = residual_correction<L>(p, amax, start, a.residual_tol, alpha, ev, cv);
-        // The network's root stands only where the reference Newton from the
-        // stored alpha provably reaches it; else the cell is deferred and
-        // plain Newton from the stored alpha decides (with the reference's
-        // alpha = 2 fallbacks).
-        if constexpr (MODE == 1)
-          accepted = accepted &&
-                     reference_reaches(cv, alpha, double(astate[cell]), a.residual_tol);
-        if (accepted) {
-          branch = 2;
-          first = true;
-        } else {
+          alpha = newton_termwise<L, REF && MODE == 6, MODE == 7>(p, stored, amax, a.residual_tol,
+                                                                  branch, its);
+      } else if constexpr (MODE == 3 || (FLAT && MODE == 4)) {
+        // alphaMax is its cap 2.5 where every |n| / f is below 0.4
+        if (!(range.x < 0.39f && range.f > 1.0e-30f) && alpha_capped<L, false>(p, alpha, amax))
+          branch = 1;
+        else
+          alpha = newton_residual<L>(p, amax, stored, a.residual_tol, branch, its);
+      } else if constexpr (SERIES) {
+        // MODE 0: the reference Newton.  MODE 4: plain Newton from the stored
+        // alpha to the residual tolerance.  MODES 1 and 2: the certified
+        // correction of the network's or of the stored alpha, and plain Newton
+        // where it does not settle the cell.
+        int outcome = SOLVE_BEYOND;
+        auto settled = [&](double x, double d) {
+          if constexpr (std::is_same_v<C, double>) return true;
+          return C(a.beta * (x - d)) == C(a.beta * (x + d)) && C(x - d) == C(x + d);
+        };
+        with_entropy_series<L>(p, range, stored, [&](const auto& s) {
+          const double gnoise = log_form_noise<L>(rho);
+          if constexpr (MODE == 0) {
+            outcome = series_newton_reference(s, stored, gnoise, alpha, its, settled);
+          } else {
+            int before = 0;
+            if constexpr (MODE != 4) {
+              EvalCurv cv{};
+              first = series_correction(s, MODE == 1 ? start : stored, a.residual_tol,
+                                        MODE == 1 ? 1 : 2, alpha, before, cv);
+              if constexpr (MODE == 1)
+                first = first && reference_reaches(cv, alpha, stored, a.residual_tol);
+            }
+            if (first)
+              outcome = SOLVE_DONE;
+            else
+              outcome = series_newton_residual(s, stored, a.residual_tol, gnoise, alpha, its,
+                                               settled);
+            its += before;
+            if (MODE != 4 && outcome == SOLVE_BEYOND) its = before;
+          }
+        });
+        if (outcome == SOLVE_BEYOND) {
           deferred = true;  // listed below, once the wavefront has reconverged
+          if constexpr (MODE == 0 || MODE == 4) its = 0;
+        } else {
+          branch = outcome == SOLVE_DONE ? 2 : 3;
+          if (outcome != SOLVE_DONE) alpha = 2.0;
         }
-        its = ev;
+      } else if constexpr (MODE == 1 || MODE == 2) {
+        // The same corrections in the log1p form (D2Q9); if the solve is not
+        // accepted plain Newton decides -- in the MODE 3 launch that follows,
+        // from the untouched stored alpha, with the reference's outcome.
+        if constexpr (MODE == 2) start = stored;
+        bool accepted = false;
+        EvalCurv cv{};
+        if (!(range.x < 0.39f && range.f > 1.0e-30f) && alpha_capped<L, false>(p, alpha, amax)) {
+          branch = 1;
+        } else {
+          accepted = residual_correction<L>(p, amax, start, a.residual_tol, alpha, its, cv);
+          if constexpr (MODE == 1)
+            accepted = accepted && reference_reaches(cv, alpha, stored, a.residual_tol);
+          if (accepted) {
+            branch = 2;
+            first = true;
+          } else {
+            deferred = true;
+          }
+        }
       }
-      // The sample log records the Newton solves: every solve in MODE 0 and
-      // MODE 4, the solves the correction deferred in MODE 3 (the cells the
-      // network or the stored alpha missed -- data to retrain on).
-      if constexpr (Shape::NIN > 0 && (MODE == 0 || MODE == 3 || MODE == 4)) {
-        if (a.log_cap > 0 && branch == 2 &&
+      // The sample log records the Newton solves: every solve of the Newton
+      // modes, of the correction modes those it deferred to MODE 3 (the cells
+      // the network or the stored alpha missed -- data to retrain on).
+      if constexpr (Shape::NIN > 0 && MODE != 1 && MODE != 2) {
+        if (a.log_cap > 0 && branch == 2 && (!groups || threadIdx.x % kGroupLanes == 0) &&
             sample_hash((unsigned)cell, a.log_salt) < a.log_threshold) {
           const unsigned long long k = atomicAdd(a.log_count, 1ull);
           if ((long long)k < a.log_cap) {
@@ -521,7 +668,14 @@ __global__ void __launch_bounds__(BLOCK)
         }
       }
     }
-    if (!deferred) {
+    // of a group the first lane speaks for the cell
+    bool speaks = !deferred;
+    if (groups && threadIdx.x % kGroupLanes != 0) {
+      speaks = false;
+      branch = -1;
+      its = 0;
+    }
+    if (speaks) {
     astate[cell] = C(alpha);  // Algorithm.h:106
     const C gc = C(a.guo_coef);
     // tau = 1 / (alpha beta); collide with 1 / tau (Collision.h:240, 254).
@@ -565,24 +719,27 @@ __global__ void __launch_bounds__(BLOCK)
     if (a.store) store_fields<L, C>(a, cell, FSX, rho, u, F, alpha);
     }
   }
-  if constexpr (MODE == 1 || MODE == 2) {
+  if constexpr (MODE == 1 || MODE == 2 || SERIES) {
     // One counter atomic per wavefront: the lanes' list slots follow from the
-    // ballot (about a quarter of the cells defer in a turbulent D3Q27 run).
+    // ballot.
     const unsigned long long mask = __ballot(deferred);
     if (mask) {
       const int lane = threadIdx.x & 63;
       const int leader = __ffsll((long long)mask) - 1;
+      const int shard = blockIdx.x % a.defer.shards;
       unsigned base = 0u;
-      if (lane == leader) base = atomicAdd(a.defer_count, (unsigned)__popcll(mask));
+      if (lane == leader)
+        base = atomicAdd(&a.defer.count[shard * kDeferStride], (unsigned)__popcll(mask));
       base = __shfl(base, leader);
       if (deferred)
-        a.defer_list[base + (unsigned)__popcll(mask & ((1ull << lane) - 1ull))] = cell;
+        a.defer.cells[(size_t)shard * a.defer.capacity + base +
+                      (unsigned)__popcll(mask & ((1ull << lane) - 1ull))] = cell;
     }
   }
   if (a.stats) {
     // a deferred cell counts its correction's evaluations here and its
-    // branch and Newton iterations in the MODE 3 launch
-    if constexpr (STRIDED) {
+    // branch and Newton iterations in the list launch
+    if constexpr (LIST) {
       // static indices only: a runtime index would put the tally in scratch
       static_for<4>([&](auto bc) {
         constexpr int b = decltype(bc)::value;
@@ -597,10 +754,10 @@ __global__ void __launch_bounds__(BLOCK)
       if (first) atomicAdd(&s_cnt[5], 1u);
     }
   }
-  if constexpr (!STRIDED) break;
+  if constexpr (!LIST) break;
   }  // list passes
   if (a.stats) {
-    if constexpr (STRIDED) {
+    if constexpr (LIST) {
       __syncthreads();
       static_for<6>([&](auto kc) {
         constexpr int k = decltype(kc)::value;

@@ -4,6 +4,8 @@
 // mode (FP64: off, for reference-order parity; FP32: fused).
 #pragma once
 
+#include <algorithm>
+
 #include "fused_step.hpp"
 #include "fused_step_vec.hpp"
 #include "registry.hpp"
@@ -21,34 +23,47 @@ hipError_t launch_step(const StepArgs& a, int fsx, int block, int grid,
       hipLaunchKernelGGL((k_bgk<L, S, C, FS, EQ, SH, 256, false>), dim3(grid),
                          dim3(block), 0, st, a, fsx);
   }
-  else if (a.alpha_mode == 0)
-    hipLaunchKernelGGL((k_elbm<L, S, C, FS, EQ, SH, 256, 0>), dim3(grid),
-                       dim3(block), 0, st, a, fsx);
-  else if (a.alpha_mode == 3)
-    // plain Newton from the stored alpha to the residual tolerance (MODE 4)
-    hipLaunchKernelGGL((k_elbm<L, S, C, FS, EQ, SH, 256, 4>), dim3(grid),
-                       dim3(block), 0, st, a, fsx);
   else {
-    // Modes 1 and 2: the certified correction, then plain Newton for the
-    // cells it deferred (MODE 3, striding over the list).
-    hipLaunchKernelGGL((k_defer_reset<0>), dim3(1), dim3(64), 0, st, a.defer_count);
-    if (a.alpha_mode == 2) {
-      hipLaunchKernelGGL((k_elbm<L, S, C, FS, EQ, SH, 256, 2>), dim3(grid),
-                         dim3(block), 0, st, a, fsx);
-    } else if constexpr (MlpShape<L>::NIN > 0) {
-      // The learned solver stages the network in LDS (dynamic shared memory).
-      using M = MfmaLayout<MlpShape<L>::NIN, MlpShape<L>::H1, MlpShape<L>::H2>;
-      hipLaunchKernelGGL((k_elbm<L, S, C, FS, EQ, SH, 256, 1>), dim3(grid),
-                         dim3(block), M::BYTES, st, a, fsx);
+    constexpr bool REF = std::is_same_v<C, double> && !SH;
+    constexpr bool FLAT = L::dimQ <= 9;
+    auto whole = [&](auto mode, size_t lds = 0) {
+      hipLaunchKernelGGL((k_elbm<L, S, C, FS, EQ, SH, 256, decltype(mode)::value>), dim3(grid),
+                         dim3(block), lds, st, a, fsx);
+    };
+    // the listed cells, or without a list every cell
+    auto listed = [&](auto mode) {
+      const int blocks =
+          a.defer.cells ? a.defer.shards * kDeferBlocks : (int)(((long long)a.N + 255) / 256);
+      hipLaunchKernelGGL((k_elbm<L, S, C, FS, EQ, SH, 256, decltype(mode)::value>), dim3(blocks),
+                         dim3(256), 0, st, a, fsx);
+    };
+    if (a.alpha_mode == 0) {
+      if constexpr (REF) {
+        whole(std::integral_constant<int, 6>{});
+      } else {
+        if (a.defer.cells) whole(std::integral_constant<int, 0>{});
+        if constexpr (FLAT) {
+          if (a.defer.cells) listed(std::integral_constant<int, 5>{});
+          else whole(std::integral_constant<int, 6>{});
+        } else {
+          listed(std::integral_constant<int, 5>{});
+        }
+      }
+    } else if (a.alpha_mode == 3) {
+      if (FLAT || a.defer.cells) whole(std::integral_constant<int, 4>{});
+      if constexpr (!FLAT) listed(std::integral_constant<int, 7>{});
     } else {
-      return hipErrorInvalidValue;
+      if (a.alpha_mode == 2) {
+        whole(std::integral_constant<int, 2>{});
+      } else if constexpr (MlpShape<L>::NIN > 0) {
+        // The learned solver stages the network in LDS (dynamic shared memory).
+        using M = MfmaLayout<MlpShape<L>::NIN, MlpShape<L>::H1, MlpShape<L>::H2>;
+        whole(std::integral_constant<int, 1>{}, M::BYTES);
+      } else {
+        return hipErrorInvalidValue;
+      }
+      listed(std::integral_constant<int, FLAT ? 3 : 7>{});
     }
-    // a capped grid striding over the list, or (log-form plain Newton) one
-    // thread per possible entry
-    const int full = (a.N + 255) / 256;
-    hipLaunchKernelGGL((k_elbm<L, S, C, FS, EQ, SH, 256, 3>),
-                       dim3(kLogResidual<L> ? full : std::min(full, kDeferBlocks)), dim3(256),
-                       0, st, a, fsx);
   }
   return hipGetLastError();
 }

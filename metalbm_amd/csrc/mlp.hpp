@@ -2,9 +2,9 @@
 //
 // No reference counterpart: the reference finds alpha by Newton only
 // (Collision.h:328-349).  Here a small ReLU MLP maps the cell's normalised
-// non-equilibrium moments to a first guess of alpha; the Newton loop below
-// (residual_correction) then certifies or corrects it, and the reference
-// Newton takes over when it cannot.
+// non-equilibrium moments to a first guess of alpha; series_correction
+// (entropy_series.hpp) then certifies or corrects it, and plain Newton from
+// the stored alpha takes over when it cannot.
 //
 // Features: m_k = (1/rho) sum_i fneq_i prod_d phi_{a_kd}(c_id), phi_0 = 1,
 // phi_1 = c, phi_2 = c^2, over the full tensor basis a_k in {0,1,2}^D (the
@@ -520,99 +520,6 @@ __device__ __forceinline__ bool residual_correction(const V& p, double amax,
   if (!(bound <= tol)) return false;
   alpha = a1;
   return true;
-}
-
-// Residual Newton with G and G' in the reference's logarithmic form
-// (EntropicStep.h:31-62): G(a) = sum f ln(f/w) - sum (f - a n) ln((f - a n)/w),
-// G'(a) = sum n (1 + ln((f - a n)/w)), one library logarithm per term, the
-// constant sum taken once.  Up to max_evals evaluations from `start`:
-// accepts the first iterate with |G| <= tol inside (1, amax) -- if STRICT,
-// also a Newton point whose Taylor remainder bound is <= tol, without
-// evaluating G there (see below); returns false
-// when an iterate leaves the evaluation interval -- (1, amax) if STRICT (the
-// certified solvers), else a > 0 with every f - a n > 0 (outside, a
-// logarithm is NaN and so is G: the reference's loop fails there too) -- or
-// max_evals evaluations do not reach tol.
-// FP64 rounding of G is ~1e-15 absolute here (terms of order 1e-2), far below
-// the tolerances used.  Fewer live values than the log1p form of
-// residual_terms (no x_i, no series variants, no curvature), which keeps the
-// D3Q27 kernels within their register budget; D2Q9 keeps the cheaper series
-// form.  evals: G evaluations made.  FRESH converts the stored populations
-// to FP64 anew in every evaluation (V::f_fresh / n_fresh) instead of letting
-// the compiler keep 2Q converted doubles live across the iterations: with
-// the certificate's terms that held the two-evaluation D3Q27 solver at 61
-// spilled registers (7 with FRESH); the one-launch plain Newton, with fewer
-// live terms, runs faster without it.
-template <class L, bool STRICT, bool FRESH, class V>
-__device__ __forceinline__ bool residual_newton_log(const V& p, double amax, double start,
-                                                    double tol, int max_evals,
-                                                    double& alpha, int& evals,
-                                                    EvalCurv& cv) {
-  constexpr int Q = L::dimQ;
-  evals = 0;
-  double SA = 0.0;
-  static_for<Q>([&](auto ic) {
-    constexpr int i = decltype(ic)::value;
-    constexpr double inv_w = 1.0 / L::W[i];
-    SA += p.template f<i>() * log(p.template f<i>() * inv_w);
-  });
-  double a = start;
-  for (int it = 0; it < max_evals; ++it) {
-    // STRICT keeps its iterates inside (1, amax); the plain Newton, like the
-    // reference's loop, bounds a only at convergence: an iterate outside the
-    // logarithms' domain gives a NaN G and ends in the fallback.
-    if (STRICT ? !(a > 1.0 && a < amax) : !(a > 0.0)) return false;
-    // STRICT: each evaluation also gathers the curvature terms of the
-    // certificate below, h = sum n^2 / fm and r = max |n| / fm, in the same
-    // pass over the populations.
-    constexpr bool cert = STRICT;
-    double g = SA, dg = 0.0, h = 0.0, r = 0.0;
-    static_for<Q>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      constexpr double inv_w = 1.0 / L::W[i];
-      double ni, fi;
-      if constexpr (FRESH) {
-        ni = p.template n_fresh<i>();
-        fi = p.template f_fresh<i>();
-      } else {
-        ni = p.template n<i>();
-        fi = p.template f<i>();
-      }
-      const double fm = fi - a * ni;
-      const double lg = log(fm * inv_w);
-      g -= fm * lg;
-      dg += ni * (1.0 + lg);
-      if constexpr (cert) {
-        const double rf = recip_refined(fm);
-        h += ni * ni * rf;
-        r = fmax(r, fabs(ni) * rf);
-      }
-    });
-    evals = it + 1;
-    cv = EvalCurv{a, dg, h, r};  // h, r: STRICT only
-    if (fabs(g) <= tol) {
-      if (!(a > 1.0 && a < amax)) return false;
-      alpha = a;
-      return true;
-    }
-    const double step = g / dg;
-    if constexpr (cert) {
-      // Certificate of the Newton point a1 = a - step without evaluating G
-      // there: G(a1) = 1/2 step^2 G''(xi) for some xi between a and a1, and
-      // f - xi n = fm + (a - xi) n >= fm (1 - |step| r) > 0, so
-      // |G''(xi)| = sum n^2 / (f - xi n) <= h / (1 - |step| r); a relative
-      // allowance of 1e-6 covers the rounding of the bound.
-      const double a1 = a - step;
-      const double room = 1.0 - fabs(step) * r;
-      if (a1 > 1.0 && a1 < amax && room > 0.0 &&
-          0.5 * step * step * h / room * (1.0 + 1e-6) <= tol) {
-        alpha = a1;
-        return true;
-      }
-    }
-    a -= step;
-  }
-  return false;
 }
 
 // Plain Newton to the residual tolerance: from `start` (the stored alpha),

@@ -37,6 +37,29 @@ namespace lbm {
 constexpr int kStatSlots = 256;
 constexpr int kStatStride = 16;  // counters per slot: 6 used, padded to 128 bytes
 
+// Cells that an entropic step's first launch does not settle, solved by a
+// second one, so that the first does not carry the other solver's registers.
+// Workgroup b appends to shard b mod `shards`, whose counter has a cache line
+// of its own and whose segment of `cells` holds every cell of its workgroups:
+// with one counter, the appends of the 86% of wavefronts that list a cell
+// (D2Q9 2048^2, reference Newton) serialised on its line and the launch took
+// 545 us instead of 150.
+struct DeferList {
+  int* cells;       // NULL: no list, the second solver takes every cell
+  unsigned* count;  // this step's counters, one per kDeferStride
+  unsigned* next;   // the next step's, which this step's second launch clears
+                    // (the first step's are cleared at the start of the call)
+  int shards, capacity;
+};
+constexpr int kDeferShards = 256;
+constexpr int kDeferStride = 32;
+constexpr int kDeferCounters = kDeferShards * kDeferStride;
+// Workgroups per shard of the second launch: with 256 shards, eight per CU,
+// enough to keep every SIMD busy at the entropic kernels' occupancy while the
+// list is long; when nothing is listed it costs little more than an empty
+// launch.
+constexpr int kDeferBlocks = 8;
+
 struct StepArgs {
   const void* src;
   void* dst;
@@ -60,8 +83,8 @@ struct StepArgs {
   unsigned long long* stats;  // ELBM counters (kStatSlots slots) or NULL
   // Entropic alpha solver: 0 reference Newton; 1 network start, 2 stored
   // alpha start, each with one certified correction (|G| <= residual_tol or
-  // Taylor bound), else the reference Newton; 3 plain Newton from the stored
-  // alpha until |G| <= residual_tol.
+  // Taylor bound), else plain Newton; 3 plain Newton from the stored alpha
+  // until |G| <= residual_tol.
   int alpha_mode;
   double residual_tol;
   const void* mlp_packed;  // network in its LDS layout (alpha mode 1)
@@ -72,11 +95,7 @@ struct StepArgs {
   long long log_cap;
   unsigned log_threshold;  // sample when hash(cell, salt) < threshold
   unsigned log_salt;
-  // Alpha modes 1 and 2: cells whose certified correction fails are listed
-  // here and solved by a second launch running plain Newton, so the
-  // correction kernel does not carry the Newton's registers.
-  unsigned* defer_count;
-  int* defer_list;  // N entries
+  DeferList defer;
 };
 
 // Storage / compute codes (values of LBM_F64 / LBM_F32 / LBM_F16).
