@@ -62,6 +62,8 @@ struct lbm_handle {
   hipStream_t stream = nullptr;
   bool own_stream = false;
   StepFn step = nullptr;
+  MarchFn march = nullptr;  // two steps in one launch (NULL: one step at a time)
+  MarchTiling tiling{};
   int64_t steps = 0;
   double w[27], scale[27];
   std::string err;
@@ -147,6 +149,31 @@ StepFn choose_kernel(const lbm_config* cfg, int* vec) {
   KernelKey kv = key;
   kv.vec = *vec;
   return registry().find(kv);
+}
+
+// The two-step kernel for the handle's domain, where it is the faster one.  Only
+// the automatic choice takes it: a caller that asks for a kernel shape gets that.
+constexpr int kMarchSlots = 256;  // one workgroup to a CU
+void choose_march(lbm_handle* h) {
+  const lbm_config& c = h->cfg;
+  if (c.collision != LBM_BGK || c.kernel != LBM_KERNEL_AUTO || h->D != 3) return;
+  const KernelKey key{c.lattice, c.collision, src_of(c.forcing_scheme), c.equilibrium,
+                      c.storage, h->ctype, c.shifted ? 1 : 0};
+  const MarchKernel k = registry().find_march(key);
+  if (!k.launch[0] || h->ffield) return;  // it reads forces from the axis tables only
+  // byte offsets within a plane are 32-bit
+  if ((double)c.ny * c.nz * (double)h->elem >= 4294967296.0) return;
+  bool side = false;
+  for (int d = 0; d < 3; ++d) side = side || (h->ftab[d] && (h->fax[d] == 1 || h->fax[d] == 2));
+  if (src_of(c.forcing_scheme) == SRC_ZERO) side = false;
+  const MarchShape m = march_shape(c.nx, c.ny, c.nz, k.columns[side], k.interior,
+                                   side ? k.side : 0, kMarchSlots, 128 / (int)h->elem);
+  const int src = src_of(c.forcing_scheme);
+  const double limit = march_limit(c.lattice == LBM_D3Q27, c.equilibrium == LBM_EQ_EXACT,
+                                   src != SRC_ZERO, src == SRC_EDM);
+  if (!march_pays(m, (double)h->N, k.interior, limit)) return;
+  h->march = k.launch[side];
+  h->tiling = MarchTiling{m.ty, m.tz, m.tiles_y, m.tiles_z, m.ranges};
 }
 
 // Force tables (Force.h:154-159, 208-215, 262-267), FP64 on the host with the
@@ -566,6 +593,7 @@ int lbm_create(const lbm_config* cfg, lbm_handle** out) {
   }
   h->own_stream = true;
   if (int rc = build_force_tables(h)) return bail(rc);
+  choose_march(h);
   if (cfg->collision == LBM_ELBM) {
     const size_t ab = (size_t)h->N * (h->ctype == TYPE_F64 ? 8 : 4);
     e = hipMalloc(&h->alpha, ab);
@@ -910,6 +938,12 @@ int lbm_step(lbm_handle* h, int nsteps, int store_last) {
   const bool field_force = h->ffield != nullptr;
   const bool time_dependent = h->cfg.force == LBM_FORCE_ENERGY_REMOVAL ||
                               h->cfg.force == LBM_FORCE_TURBULENT_2D;
+  // Steps taken two to a launch: an even number of pairs, so that the populations
+  // end in the same lattice as after one launch a step (a captured graph of an
+  // even number of steps then starts its replays where it ended, and so does a
+  // caller that keeps lbm_device_populations across them), and never the storing
+  // step.
+  int paired = h->march ? (nsteps - (store_last ? 1 : 0)) / 4 * 4 : 0;
   for (int s = 0; s < nsteps; ++s) {
     // Collision::update before the step (Algorithm.h:338, Collision.h:96-99);
     // ConstantShell is set once (Collision.h:51-54).  EnergyRemoval and
@@ -935,6 +969,15 @@ int lbm_step(lbm_handle* h, int nsteps, int store_last) {
       a.uh_out = h->fields + h->N;
       a.alpha_out = h->fields + (size_t)h->N * (1 + h->D);
       a.F_out = h->fields + (size_t)h->N * (2 + h->D);
+    }
+    if (paired > 0) {
+      const hipError_t e = h->march(a, h->tiling, h->stream);
+      if (e != hipSuccess) return hip_fail(h, e, "two-step launch");
+      h->cur = 1 - h->cur;
+      h->steps += 2;
+      paired -= 2;
+      ++s;
+      continue;
     }
     hipError_t e = h->step(a, h->cfg.forcing_scheme, h->block, grid, h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "fused step launch");

@@ -179,4 +179,70 @@ int pick_vector_width(const lbm_config* cfg, F&& instantiated) {
   return 0;
 }
 
+// Tiling of the two-step kernel: tiles of ty x tz columns and a split of the x
+// extent into ranges, for a kernel that holds `columns` columns with the rim and
+// `interior` without, force tables of `side` rows or places (0: none needed),
+// `slots` workgroups running at once and `line` values to a cache line.  cost
+// estimates the time of a launch in units of one pass over the lattice: the
+// writes, the reads (rows of the rim, whole lines at the ends of split rows, two
+// planes for each range) and a fixed time per plane (a least-squares fit over 15
+// shapes of eight configurations gives it as 0.35 to 1.2 of the time that
+// `interior` columns take; residuals of 4 to 12 %), over the share of the slots
+// that is busy.
+// ranges == 0: nothing fits.
+struct MarchShape {
+  int ty = 0, tz = 0, tiles_y = 0, tiles_z = 0, ranges = 0;
+  double cost = 0.0;
+};
+inline MarchShape march_shape(int nx, int ny, int nz, int columns, int interior, int side,
+                              int slots, int line) {
+  MarchShape best;
+  // splits of the rows from the longest parts that fit, down to about a line
+  const int first = (nz + interior - 1) / interior;
+  for (int parts = first; parts <= (nz + 31) / 32 && parts < first + 64; ++parts) {
+    const int tz = (nz + parts - 1) / parts, kz = (nz + tz - 1) / tz;
+    const int pitch = kz == 1 ? tz : tz + 2;
+    if (tz > interior || 3 * pitch > columns || (side && pitch > side) || pitch > 32767) continue;
+    int ty = columns / pitch - 2;
+    if (ty > interior / tz) ty = interior / tz;
+    if (side && ty > side - 2) ty = side - 2;
+    if (ty > ny) ty = ny;
+    if (ty < 1) continue;
+    int ky = (ny + ty - 1) / ty;
+    ty = (ny + ky - 1) / ky;
+    ky = (ny + ty - 1) / ty;
+    const long long tiles = (long long)ky * kz;
+    const double lines = (double)((tz + line - 1) / line);
+    const double rows = (double)(ty + 2) * ky / ny * (kz == 1 ? 1.0 : (lines + 2.0) / lines);
+    for (int r = 1; r <= nx; ++r) {
+      const long long rounds = (tiles * r + slots - 1) / slots;
+      if (r > 1 && rounds > 32) break;
+      const int len = (nx + r - 1) / r;
+      const double busy = (double)tiles * nx / ((double)rounds * slots * len);
+      const double fixed = 0.75 * interior * (double)tiles / ((double)ny * nz);
+      const double cost = (1.0 + (rows + fixed) * (len + 2) / len) / busy;
+      if (best.ranges == 0 || cost < best.cost) best = MarchShape{ty, tz, ky, kz, r, cost};
+    }
+  }
+  return best;
+}
+
+// Whether that tiling beats two one-step launches, from 21 shapes of at least
+// 2^18 cells under eleven combinations of lattice, equilibrium, source and force
+// (FP32).  Below the limits the two-step kernel took 0.13 to 1.00 of the one-step
+// kernel's time; above them up to 1.5 of it: the more a collision computes (a
+// product equilibrium with a source, the exact-difference source's second
+// equilibrium), the less the rim's second collision may cost.  D3Q19's one-step
+// kernel is slow on small domains (64^3: 19.2 us a step, two-step 13.0; D3Q27: 12.6
+// and 12.7).  Tiles that fill less than half of the kernel's columns (2048 x 16 x 16)
+// leave lanes idle.
+inline double march_limit(bool q27, bool exact, bool source, bool difference) {
+  if (exact && source) return 3.9;
+  if (q27) return 6.1;
+  return difference ? 5.3 : 13.0;
+}
+inline bool march_pays(const MarchShape& m, double cells, int interior, double limit) {
+  return m.ranges > 0 && cells >= 262144.0 && 2 * m.ty * m.tz >= interior && m.cost <= limit;
+}
+
 }  // namespace lbm

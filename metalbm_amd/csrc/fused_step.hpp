@@ -36,25 +36,124 @@ __device__ __forceinline__ void store_fields(const StepArgs& a, int cell, int FS
     for (int d = 0; d < L::dimD; ++d) a.F_out[(size_t)d * a.N + cell] = double(F[d]);
 }
 
-// FSX: the forcing scheme as configured (None vs Shan-Chen matters only for
-// the stored hydrodynamic velocity), passed at run time.
-// NT: non-temporal population loads (chosen per configuration by the host).
-template <class L, class S, class C, int FS, int EQ, bool SH, int BLOCK, bool NT>
-__global__ void __launch_bounds__(BLOCK) k_bgk(const StepArgs a, int FSX) {
+// Index of the population with the opposite velocity.
+template <class L, int i>
+constexpr int opposite() {
+  for (int j = 0; j < L::dimQ; ++j) {
+    bool opp = true;
+    for (int d = 0; d < L::dimD; ++d) opp = opp && L::C[j][d] == -L::C[i][d];
+    if (opp) return j;
+  }
+  return -1;
+}
+
+// Coefficients of scale (base + rho (P(cu) - 1)), P the Ma3 polynomial, split into
+// its even part e0 + cu^2 (e1 + e2 cu^2) and its odd part cu (o0 + o1 cu^2).
+struct Ma3Split {
+  float e0, e1, e2, o0, o1;
+  __device__ __forceinline__ Ma3Split(float scale, float rho, float base, float u2) {
+#pragma clang fp contract(off)
+    const float sr = scale * rho;
+    e0 = fmaf(sr, u2 * fmaf(1.125f, u2, -1.5f), scale * base);
+    e1 = sr * fmaf(-6.75f, u2, 4.5f);
+    e2 = sr * 3.375f;
+    o0 = sr * fmaf(-4.5f, u2, 3.0f);
+    o1 = sr * 4.5f;
+  }
+  __device__ __forceinline__ float even(float q, float more) const {
+    return fmaf(q, fmaf(q, e2, e1), more);
+  }
+  __device__ __forceinline__ float odd(float cu, float q, float more) const {
+    return fmaf(cu, fmaf(q, o1, o0), more);
+  }
+};
+
+// The single-precision Ma3 collision, two opposite populations at a time: they
+// share every term of the equilibrium and of the source up to the sign of the
+// odd part, and the relaxation rate and the source are folded into the
+// polynomial's coefficients once per cell (the two-step kernel on D3Q19 256^3 with
+// the Guo source: 179 million vector instructions a launch instead of 248, addresses
+// included).  Contraction is off and every fused operation is written out, so each
+// kernel that inlines this gets the same bits.
+template <class L, int FS, bool SH, class EMIT>
+__device__ __forceinline__ void bgk_collide_pairs(const StepArgs& a, const float* f,
+                                                  const float* F, float& rho, float* u,
+                                                  EMIT&& emit) {
+#pragma clang fp contract(off)
+  constexpr int Q = L::dimQ, D = L::dimD;
+  const float of = float(a.omega_f), oe = float(a.omega_eq), g3 = float(3.0 * a.guo_coef);
+  float sum = f[0], j[3] = {0.0f, 0.0f, 0.0f};
+  static_for<Q>([&](auto ic) {
+    constexpr int i = decltype(ic)::value, o = opposite<L, i>();
+    if constexpr (i < o) {
+      sum += f[i] + f[o];
+      const float d = f[i] - f[o];
+      static_for<D>([&](auto dc) {
+        constexpr int c = L::C[i][decltype(dc)::value];
+        if constexpr (c > 0) j[decltype(dc)::value] += d;
+        if constexpr (c < 0) j[decltype(dc)::value] -= d;
+      });
+    }
+  });
+  rho = SH ? 1.0f + sum : sum;
+  const float r0 = __builtin_amdgcn_rcpf(rho);
+  const float rr = fmaf(r0, fmaf(-rho, r0, 1.0f), r0);  // see moments_shifted_scaled
+  u[2] = 0.0f;
+  for (int d = 0; d < D; ++d) u[d] = j[d] * rr;
+  auto square = [&](const float* v) {
+    float s = v[0] * v[0];
+    for (int d = 1; d < D; ++d) s = fmaf(v[d], v[d], s);
+    return s;
+  };
+  // EDM: omega_eq feq(u) + (feq(u + F / rho) - feq(u)) (ForcingScheme.h:184-197)
+  const float scale = FS == SRC_EDM ? float(a.omega_eq - 1.0) : oe;
+  Ma3Split E(scale, rho, sum, square(u));
+  float v[3] = {0.0f, 0.0f, 0.0f};
+  if constexpr (FS == SRC_EDM)
+    for (int d = 0; d < D; ++d) v[d] = fmaf(F[d], rr, u[d]);
+  const Ma3Split E2(1.0f, rho, sum, square(v));
+  // Guo: w 3 g (c.F - u.F + 3 (c.u) (c.F)), g = 1 - 1 / (2 tau) (ForcingScheme.h:99-117)
+  float G[3] = {0.0f, 0.0f, 0.0f};
+  if constexpr (FS == SRC_GUO) {
+    for (int d = 0; d < D; ++d) G[d] = g3 * F[d];
+    for (int d = 0; d < D; ++d) E.e0 = fmaf(-u[d], G[d], E.e0);
+  }
+  if constexpr (FS == SRC_EDM) E.e0 += E2.e0;
+  emit(std::integral_constant<int, 0>{}, fmaf(float(L::W[0]), E.e0, of * f[0]));
+  static_for<Q>([&](auto ic) {
+    constexpr int i = decltype(ic)::value, o = opposite<L, i>();
+    if constexpr (i < o) {
+      constexpr float w = float(L::W[i]);
+      const float cu = cdot<L, i>(u), q = cu * cu;
+      float even = E.even(q, E.e0), odd;
+      if constexpr (FS == SRC_GUO) {
+        const float cG = cdot<L, i>(G);
+        even = fmaf(3.0f * cu, cG, even);
+        odd = E.odd(cu, q, cG);
+      } else if constexpr (FS == SRC_EDM) {
+        const float cv = cdot<L, i>(v), r = cv * cv;
+        even = E2.even(r, even);
+        odd = E.odd(cu, q, cv * fmaf(r, E2.o1, E2.o0));
+      } else {
+        odd = cu * fmaf(q, E.o1, E.o0);
+      }
+      emit(std::integral_constant<int, i>{}, fmaf(w, even + odd, of * f[i]));
+      emit(std::integral_constant<int, o>{}, fmaf(w, even - odd, of * f[o]));
+    }
+  });
+}
+
+// BGK collision of one cell (Collision.h:134-151): f the pulled populations, F the
+// force.  emit(i, v) takes the post-collision populations in order, v in the
+// compute type (f_i - w_i when SH); rho and u are the moments.
+template <class L, class C, int FS, int EQ, bool SH, class EMIT>
+__device__ __forceinline__ void bgk_collide(const StepArgs& a, const C* f, const C* F, C& rho,
+                                            C* u, EMIT&& emit) {
   constexpr int Q = L::dimQ;
   constexpr bool REF = std::is_same_v<C, double> && !SH;
-  const CellPos c = cell_of_thread<L, BLOCK>(a);
-  if (!c.active) return;
-  const int cell = self_index<L>(a, c);
-  S* __restrict__ dst = static_cast<S*>(a.dst);
-
-  C f[Q];
-  pull<L, S, C, NT>(a, c, f);
-  C F[3];
-  force_of_cell<L, C>(a, c, F);
   const C of = C(a.omega_f), oe = C(a.omega_eq), gc = C(a.guo_coef);
-  C rho, u[3] = {C(0), C(0), C(0)}, u2;
-
+  u[0] = u[1] = u[2] = C(0);
+  C u2;
   if constexpr (REF) {
     // calculateMoments (Collision.h:72-79)
     moments_ref<L>(f, rho, u, u2);
@@ -68,15 +167,13 @@ __global__ void __launch_bounds__(BLOCK) k_bgk(const StepArgs a, int FSX) {
       for (int d = 1; d < L::dimD; ++d) v2 += v[d] * v[d];
     }
     const RefEquilibrium<L, EQ, C> E2(rho, v, v2);
-    // BGK collideAndStream (Collision.h:134-151)
     static_for<Q>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
       const C fe = E.template feq<i>();
       C s = C(0);
       if constexpr (FS == SRC_GUO) s = guo_ref<L, i>(gc, u, F);
       if constexpr (FS == SRC_EDM) s = E2.template feq<i>() - fe;
-      const C out = of * f[i] + oe * fe + s;
-      store_pop<L, i, S, C>(dst + (size_t)i * a.N + cell, out);
+      emit(ic, of * f[i] + oe * fe + s);
     });
   } else {
     C drho;
@@ -110,10 +207,31 @@ __global__ void __launch_bounds__(BLOCK) k_bgk(const StepArgs a, int FSX) {
         s = (C(3) * gc * w) * (cF - uF + C(3) * cu * cF);
       }
       if constexpr (FS == SRC_EDM) s = rho * w * (E2.template p<i>() - p);
-      const C out = of * f[i] + oe * eq + s;
-      store_pop<L, i, S, C>(dst + (size_t)i * a.N + cell, out);
+      emit(ic, of * f[i] + oe * eq + s);
     });
   }
+}
+
+// FSX: the forcing scheme as configured (None vs Shan-Chen matters only for
+// the stored hydrodynamic velocity), passed at run time.
+// NT: non-temporal population loads (chosen per configuration by the host).
+template <class L, class S, class C, int FS, int EQ, bool SH, int BLOCK, bool NT>
+__global__ void __launch_bounds__(BLOCK) k_bgk(const StepArgs a, int FSX) {
+  constexpr int Q = L::dimQ;
+  const CellPos c = cell_of_thread<L, BLOCK>(a);
+  if (!c.active) return;
+  const int cell = self_index<L>(a, c);
+  S* __restrict__ dst = static_cast<S*>(a.dst);
+
+  C f[Q];
+  pull<L, S, C, NT>(a, c, f);
+  C F[3];
+  force_of_cell<L, C>(a, c, F);
+  C rho, u[3];
+  bgk_collide<L, C, FS, EQ, SH>(a, f, F, rho, u, [&](auto ic, C v) {
+    constexpr int i = decltype(ic)::value;
+    store_pop<L, i, S, C>(dst + (size_t)i * a.N + cell, v);
+  });
   if (a.store) store_fields<L, C>(a, cell, FSX, rho, u, F, 2.0);
 }
 

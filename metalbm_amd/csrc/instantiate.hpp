@@ -6,6 +6,7 @@
 
 #include <algorithm>
 
+#include "fused_march.hpp"
 #include "fused_step.hpp"
 #include "fused_step_vec.hpp"
 #include "registry.hpp"
@@ -77,6 +78,29 @@ hipError_t launch_step_vec(const StepArgs& a, int fsx, int block, int grid,
   return hipGetLastError();
 }
 
+template <class L, class S, class C, int FS, int EQ, bool SH, bool SIDE>
+hipError_t launch_march(const StepArgs& a, const MarchTiling& m, hipStream_t st) {
+  hipLaunchKernelGGL((k_bgk_march<L, S, C, FS, EQ, SH, SIDE>),
+                     dim3(m.tiles_y * m.tiles_z * m.ranges), dim3(kMarchThreads), 0, st, a, m);
+  return hipGetLastError();
+}
+template <class L, class S, class C, int FS, int EQ, bool SH>
+MarchKernel march_kernel() {
+  MarchKernel k;
+  k.launch[0] = &launch_march<L, S, C, FS, EQ, SH, false>;
+  k.columns[0] = kMarchColumns<L, S, C, false>;
+  if constexpr (FS != SRC_ZERO) {
+    k.launch[1] = &launch_march<L, S, C, FS, EQ, SH, true>;
+    k.columns[1] = kMarchColumns<L, S, C, true>;
+  } else {  // no source: the force does not enter the step
+    k.launch[1] = k.launch[0];
+    k.columns[1] = k.columns[0];
+  }
+  k.interior = kMarchUnits<L> * kMarchThreads;
+  k.side = kMarchSide;
+  return k;
+}
+
 template <class L, class S, class C, bool SH, int... Vs>
 void register_combo(Registry& r, int storage, int compute) {
   auto add_eq = [&](auto eqc) {
@@ -85,6 +109,9 @@ void register_combo(Registry& r, int storage, int compute) {
       constexpr int FS = decltype(fsc)::value;
       r.add({(int)L::Type, (int)CollisionType::BGK, FS, EQ, storage, compute, SH, 0},
             &launch_step<L, S, C, FS, EQ, SH, (int)CollisionType::BGK>);
+      if constexpr (L::dimD == 3 && std::is_same_v<S, float> && std::is_same_v<C, float>)
+        r.add({(int)L::Type, (int)CollisionType::BGK, FS, EQ, storage, compute, SH, 0},
+              march_kernel<L, S, C, FS, EQ, SH>());
       r.add({(int)L::Type, (int)CollisionType::ELBM, FS, EQ, storage, compute, SH, 0},
             &launch_step<L, S, C, FS, EQ, SH, (int)CollisionType::ELBM>);
       (r.add({(int)L::Type, (int)CollisionType::BGK, FS, EQ, storage, compute, SH, Vs},

@@ -19,6 +19,16 @@ namespace lbm {
 using StepFn = hipError_t (*)(const StepArgs&, int fsx, int block,
                               int grid, hipStream_t);
 
+// The two-step kernel of a configuration, [1] with tables for forces that vary
+// along y or z, and what its tiling has to fit: columns of a tile with its rim,
+// interior columns, entries of a force table.
+using MarchFn = hipError_t (*)(const StepArgs&, const MarchTiling&, hipStream_t);
+struct MarchKernel {
+  MarchFn launch[2] = {nullptr, nullptr};
+  int columns[2] = {0, 0};
+  int interior = 0, side = 0;
+};
+
 // vec = 0 selects the one-cell-per-lane kernel; vec = V > 0 the kernel in
 // which each lane owns V consecutive cells (aligned vector accesses).
 struct KernelKey {
@@ -31,6 +41,12 @@ struct KernelKey {
 
 struct Registry {
   std::map<int64_t, StepFn> step;
+  std::map<int64_t, MarchKernel> march;  // by the key of the one-cell-per-lane kernel
+  void add(const KernelKey& k, const MarchKernel& f) { march[k.code()] = f; }
+  MarchKernel find_march(const KernelKey& k) const {
+    auto it = march.find(k.code());
+    return it == march.end() ? MarchKernel{} : it->second;
+  }
   void add(const KernelKey& k, StepFn f) { step[k.code()] = f; }
   StepFn find(const KernelKey& k) const {
     auto it = step.find(k.code());

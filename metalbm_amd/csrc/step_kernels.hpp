@@ -98,6 +98,12 @@ struct StepArgs {
   DeferList defer;
 };
 
+// Tiling of the two-step kernel (fused_march.hpp): tiles of ty x tz columns, the
+// x extent in `ranges` parts, one workgroup for each tile and range.
+struct MarchTiling {
+  int ty, tz, tiles_y, tiles_z, ranges;
+};
+
 // Storage / compute codes (values of LBM_F64 / LBM_F32 / LBM_F16).
 enum : int { TYPE_F64 = 0, TYPE_F32 = 1, TYPE_F16 = 2 };
 
@@ -140,13 +146,16 @@ __device__ __forceinline__ C to_compute(S v) {
 }
 
 template <class L, int i, class S, class C>
+__device__ __forceinline__ S to_storage(C v) {
+  if constexpr (std::is_same_v<S, _Float16>)
+    return _Float16(float(v * C(kHalfScale<L, i>)));
+  else
+    return S(v);
+}
+
+template <class L, int i, class S, class C>
 __device__ __forceinline__ void store_pop(S* p, C v) {
-  if constexpr (std::is_same_v<S, _Float16>) {
-    const _Float16 h = _Float16(float(v * C(kHalfScale<L, i>)));
-    __builtin_nontemporal_store(h, p);
-  } else {
-    __builtin_nontemporal_store(S(v), p);
-  }
+  __builtin_nontemporal_store(to_storage<L, i, S, C>(v), p);
 }
 
 // Coordinates of the thread's cell and its periodic neighbours.

@@ -1,0 +1,54 @@
+// march_rules.cpp -- the tiling of the two-step kernel against what the kernel
+// assumes, for extents from degenerate to huge (built and run by
+// tests/test_march_rules.py).  Prints, for the extents given as arguments, whether
+// the automatic choice takes the two-step kernel.
+#include <cstdio>
+#include <cstdlib>
+
+#include "config_rules.hpp"
+
+static int failures = 0;
+static void check(bool ok, const char* what, int nx, int ny, int nz, int columns) {
+  if (ok) return;
+  std::printf("FAIL %s at %d x %d x %d, %d columns\n", what, nx, ny, nz, columns);
+  ++failures;
+}
+
+// (columns, interior, side) of D3Q19 and D3Q27 in FP32, without and with force tables
+static const int kernels[4][3] = {
+    {2560, 2048, 0}, {2510, 2048, 264}, {1704, 1024, 0}, {1672, 1024, 264}};
+
+int main(int argc, char** argv) {
+  if (argc == 6) {  // nx ny nz kernel limit
+    const int* k = kernels[std::atoi(argv[4])];
+    const int nx = std::atoi(argv[1]), ny = std::atoi(argv[2]), nz = std::atoi(argv[3]);
+    const lbm::MarchShape m = lbm::march_shape(nx, ny, nz, k[0], k[1], k[2], 256, 32);
+    std::printf("%d\n", (int)lbm::march_pays(m, (double)nx * ny * nz, k[1], std::atof(argv[5])));
+    return 0;
+  }
+  const int extents[] = {1,   2,   3,   7,    8,    9,    31,   32,   33,    64,     96,
+                         130, 161, 256, 257,  263,  264,  265,  511,  512,   513,    1000,
+                         1025, 2047, 2048, 2049, 2561, 8193, 65537, 1000003};
+  int shapes = 0;
+  for (const auto& k : kernels)
+    for (int nx : {1, 2, 3, 17, 256, 1000})
+      for (int ny : extents)
+        for (int nz : extents) {
+          if ((double)ny * nz * 4.0 >= 4294967296.0) continue;
+          const lbm::MarchShape m = lbm::march_shape(nx, ny, nz, k[0], k[1], k[2], 256, 32);
+          if (m.ranges == 0) continue;
+          ++shapes;
+          auto ok = [&](bool c, const char* what) { check(c, what, nx, ny, nz, k[0]); };
+          const long long pitch = m.tiles_z == 1 ? m.tz : m.tz + 2;
+          ok(m.ty >= 1 && m.tz >= 1 && m.ranges >= 1 && m.ranges <= nx, "positive");
+          ok((long long)m.ty * m.tiles_y >= ny && (long long)m.ty * (m.tiles_y - 1) < ny, "rows");
+          ok((long long)m.tz * m.tiles_z >= nz && (long long)m.tz * (m.tiles_z - 1) < nz, "places");
+          ok((m.ty + 2) * pitch <= k[0], "columns in LDS");
+          ok((long long)m.ty * m.tz <= k[1], "columns in registers");
+          ok(m.ty + 1 < 32768 && pitch <= 32767, "packed column index");
+          if (k[2]) ok(m.ty + 2 <= k[2] && pitch <= k[2], "force tables");
+          ok((long long)m.tiles_y * m.tiles_z * m.ranges < (1ll << 31), "grid");
+        }
+  std::printf("%d shapes, %d failures\n", shapes, failures);
+  return failures != 0 || shapes < 2000;
+}
