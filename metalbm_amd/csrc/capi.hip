@@ -169,8 +169,9 @@ void choose_march(lbm_handle* h) {
   const MarchShape m = march_shape(c.nx, c.ny, c.nz, k.columns[side], k.interior,
                                    side ? k.side : 0, kMarchSlots, 128 / (int)h->elem);
   const int src = src_of(c.forcing_scheme);
-  const double limit = march_limit(c.lattice == LBM_D3Q27, c.equilibrium == LBM_EQ_EXACT,
-                                   src != SRC_ZERO, src == SRC_EDM);
+  const double limit =
+      march_limit(h->ctype == TYPE_F64, c.lattice == LBM_D3Q27, c.equilibrium == LBM_EQ_EXACT,
+                  src != SRC_ZERO, src == SRC_EDM);
   if (!march_pays(m, (double)h->N, k.interior, limit)) return;
   h->march = k.launch[side];
   h->tiling = MarchTiling{m.ty, m.tz, m.tiles_y, m.tiles_z, m.ranges};

@@ -227,16 +227,17 @@ inline MarchShape march_shape(int nx, int ny, int nz, int columns, int interior,
   return best;
 }
 
-// Whether that tiling beats two one-step launches, from 21 shapes of at least
-// 2^18 cells under eleven combinations of lattice, equilibrium, source and force
-// (FP32).  Below the limits the two-step kernel took 0.13 to 1.00 of the one-step
+// Whether that tiling beats two one-step launches, from 15 to 21 shapes of at least
+// 2^18 cells under 19 combinations of lattice, equilibrium, source, force and number
+// format.  Below the limits the two-step kernel took 0.13 to 1.00 of the one-step
 // kernel's time; above them up to 1.5 of it: the more a collision computes (a
 // product equilibrium with a source, the exact-difference source's second
-// equilibrium), the less the rim's second collision may cost.  D3Q19's one-step
-// kernel is slow on small domains (64^3: 19.2 us a step, two-step 13.0; D3Q27: 12.6
-// and 12.7).  Tiles that fill less than half of the kernel's columns (2048 x 16 x 16)
-// leave lanes idle.
-inline double march_limit(bool q27, bool exact, bool source, bool difference) {
+// equilibrium, FP64), the less the rim's second collision may cost.  D3Q19's
+// one-step kernel is slow on small domains (64^3: 19.2 us a step, two-step 13.0;
+// D3Q27: 12.6 and 12.7).  Tiles that fill less than half of the kernel's columns (2048 x
+// 16 x 16) leave lanes idle.
+inline double march_limit(bool fp64, bool q27, bool exact, bool source, bool difference) {
+  if (fp64) return 4.9;
   if (exact && source) return 3.9;
   if (q27) return 6.1;
   return difference ? 5.3 : 13.0;

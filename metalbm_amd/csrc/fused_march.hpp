@@ -31,9 +31,12 @@
 // Measured, microseconds a step, one-step kernels -> this one: D3Q19 256^3 456 ->
 // 257 (1.46 GB read and 1.28 GB written by a launch of 513 us, 5.3 TB/s; 64 % of
 // the vector issue slots), D3Q27 193 x 161 x 130 Ma3 260 -> 159, product
-// equilibrium 276 -> 183.  FP64 (304 against 258 at D3Q19 171 x 150 x 133: twice
-// the registers, one column a thread) and FP16 (1245 against 1211 at D3Q27 384^3:
-// as many vector instructions for half the bytes) stay with the one-step kernels.
+// equilibrium 276 -> 183; FP64, one column a thread: D3Q19 192^3 424 -> 328, 171 x
+// 150 x 133 257 -> 208 (60 % of the issue slots: before opposite populations shared
+// their terms 246, with divisions by 6 and 24 304).  FP16 (1245 against 1211 at D3Q27
+// 384^3: as many vector instructions for half the bytes) stays with the one-step
+// kernels, and so does FP64 storage with FP32 arithmetic, whose populations would
+// show that the two kernels round their FP32 sums differently.
 #pragma once
 
 #include "fused_step.hpp"
@@ -47,9 +50,10 @@ template <class L, class S, class C, bool SIDE>
 constexpr int kMarchColumns = (kMarchLds - (SIDE ? 3 * kMarchSide * int(sizeof(C)) : 0)) /
                               ((L::dimQ - 3) * int(sizeof(S))) / 4 * 4;
 // Interior columns per thread, and how many of them have pulls in flight.
-template <class L>
-constexpr int kMarchUnits = L::dimQ > 19 ? 2 : 4;
-constexpr int kMarchAhead = 2;
+template <class L, class S>
+constexpr int kMarchUnits = sizeof(S) == 8 ? 1 : (L::dimQ > 19 ? 2 : 4);
+template <class L, class S>
+constexpr int kMarchAhead = kMarchUnits<L, S> == 1 ? 1 : 2;
 
 // LDS slot of population i among those with (c_y, c_z) != 0, or -1.
 template <class L, int i>
@@ -79,8 +83,8 @@ template <class L, class S, class C, int FS, int EQ, bool SH, bool SIDE>
 __global__ void __launch_bounds__(kMarchThreads)
     __attribute__((amdgpu_waves_per_eu(2)))
     k_bgk_march(const StepArgs a, const MarchTiling m) {
-  constexpr int Q = L::dimQ, U = kMarchUnits<L>, THREADS = kMarchThreads;
-  constexpr int AHEAD = kMarchAhead;
+  constexpr int Q = L::dimQ, U = kMarchUnits<L, S>, THREADS = kMarchThreads;
+  constexpr int AHEAD = kMarchAhead<L, S>;
   static_assert(U % AHEAD == 0, "a plane's first columns find their registers free");
   constexpr int COLUMNS = kMarchColumns<L, S, C, SIDE>;
   __shared__ S lds[(Q - 3) * COLUMNS];

@@ -167,13 +167,24 @@ __device__ __forceinline__ void bgk_collide(const StepArgs& a, const C* f, const
       for (int d = 1; d < L::dimD; ++d) v2 += v[d] * v[d];
     }
     const RefEquilibrium<L, EQ, C> E2(rho, v, v2);
-    static_for<Q>([&](auto ic) {
+    auto relax = [&](auto ic, C fe, C fe2) {
       constexpr int i = decltype(ic)::value;
-      const C fe = E.template feq<i>();
       C s = C(0);
       if constexpr (FS == SRC_GUO) s = guo_ref<L, i>(gc, u, F);
-      if constexpr (FS == SRC_EDM) s = E2.template feq<i>() - fe;
+      if constexpr (FS == SRC_EDM) s = fe2 - fe;
       emit(ic, of * f[i] + oe * fe + s);
+    };
+    static_for<Q>([&](auto ic) {
+      constexpr int i = decltype(ic)::value, o = opposite<L, i>();
+      if constexpr (EQ != (int)EquilibriumType::TruncationMa3 || i == o) {
+        relax(ic, E.template feq<i>(), FS == SRC_EDM ? E2.template feq<i>() : C(0));
+      } else if constexpr (i < o) {
+        C fe, fo, ge = C(0), go = C(0);
+        feq_ma3_ref_pair<L, i>(rho, u, u2, fe, fo);
+        if constexpr (FS == SRC_EDM) feq_ma3_ref_pair<L, i>(rho, v, v2, ge, go);
+        relax(ic, fe, ge);
+        relax(std::integral_constant<int, o>{}, fo, go);
+      }
     });
   } else {
     C drho;

@@ -96,7 +96,7 @@ MarchKernel march_kernel() {
     k.launch[1] = k.launch[0];
     k.columns[1] = k.columns[0];
   }
-  k.interior = kMarchUnits<L> * kMarchThreads;
+  k.interior = kMarchUnits<L, S> * kMarchThreads;
   k.side = kMarchSide;
   return k;
 }
@@ -109,7 +109,12 @@ void register_combo(Registry& r, int storage, int compute) {
       constexpr int FS = decltype(fsc)::value;
       r.add({(int)L::Type, (int)CollisionType::BGK, FS, EQ, storage, compute, SH, 0},
             &launch_step<L, S, C, FS, EQ, SH, (int)CollisionType::BGK>);
-      if constexpr (L::dimD == 3 && std::is_same_v<S, float> && std::is_same_v<C, float>)
+      // FP64 arithmetic on D3Q27 gains without a source only (192^3 a step: 615 ->
+      // 504 us; with Guo's 616 -> 844, with the product equilibrium 608 -> 868: its
+      // registers spill).
+      constexpr bool HEAVY = std::is_same_v<C, double> && L::dimQ > 19 &&
+                             (FS != SRC_ZERO || EQ != (int)EquilibriumType::TruncationMa3);
+      if constexpr (L::dimD == 3 && std::is_same_v<S, C> && !HEAVY)
         r.add({(int)L::Type, (int)CollisionType::BGK, FS, EQ, storage, compute, SH, 0},
               march_kernel<L, S, C, FS, EQ, SH>());
       r.add({(int)L::Type, (int)CollisionType::ELBM, FS, EQ, storage, compute, SH, 0},

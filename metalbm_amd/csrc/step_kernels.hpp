@@ -267,10 +267,16 @@ template <class L, int i, class T>
 __device__ __forceinline__ T guo_ref(T gcoef, const T* u, const T* F) {
   const T cu = cdot<L, i>(u);
   const T s3 = T(3.0) * cu;
-  T r = ((T(cel<L, i, 0>()) - u[0]) + T(cel<L, i, 0>()) * s3) * F[0];
-  r += ((T(cel<L, i, 1>()) - u[1]) + T(cel<L, i, 1>()) * s3) * F[1];
-  if constexpr (L::dimD == 3)
-    r += ((T(cel<L, i, 2>()) - u[2]) + T(cel<L, i, 2>()) * s3) * F[2];
+  // (c_d - u_d) + c_d 3 (c.u)
+  auto term = [&](auto dc) {
+    constexpr int d = decltype(dc)::value, c = cel<L, i, d>();
+    if constexpr (c == 0) return -u[d];
+    else if constexpr (c > 0) return (T(1) - u[d]) + s3;
+    else return (T(-1) - u[d]) - s3;
+  };
+  T r = term(std::integral_constant<int, 0>{}) * F[0];
+  r += term(std::integral_constant<int, 1>{}) * F[1];
+  if constexpr (L::dimD == 3) r += term(std::integral_constant<int, 2>{}) * F[2];
   return gcoef * T(L::W[i]) * T(3.0) * r;
 }
 

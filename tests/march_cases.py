@@ -2,7 +2,8 @@
 that divide the domain and ragged ones, one range and many, a two-plane domain,
 one row of tiles that is its own neighbour; each source, force axis, equilibrium
 and number format."""
-from metalbm_amd import EquilibriumType, ForceType, ForcingSchemeType, LatticeType
+from metalbm_amd import (EquilibriumType, ForceType, ForcingSchemeType, LatticeType,
+                         Precision)
 
 Q19, Q27 = LatticeType.D3Q19, LatticeType.D3Q27
 MA3, EXACT = EquilibriumType.TruncationMa3, EquilibriumType.Exact
@@ -11,9 +12,13 @@ NONE, GUO, EDM = (ForcingSchemeType.None_, ForcingSchemeType.Guo,
 F = ForceType
 
 
-def case(lattice, shape, scheme, force, equilibrium, shifted):
+# storage, compute
+F32, F64 = (Precision.F32, Precision.F32), (Precision.F64, Precision.F64)
+
+
+def case(lattice, shape, scheme, force, equilibrium, shifted, numbers=F32):
     return dict(lattice=lattice, shape=shape, scheme=scheme, force=force,
-                equilibrium=equilibrium, shifted=shifted)
+                equilibrium=equilibrium, shifted=shifted, numbers=numbers)
 
 
 CASES = [
@@ -26,13 +31,22 @@ CASES = [
     case(Q27, (129, 127, 127), EDM, F.Constant, EXACT, False),
     case(Q27, (29, 70, 530), EDM, F.Sinusoidal, MA3, True),
     case(Q27, (512, 32, 33), NONE, F.None_, EXACT, True),
+    case(Q19, (71, 90, 77), GUO, F.Kolmogorov, MA3, False, F64),
+    case(Q19, (90, 70, 301), EDM, F.Sinusoidal, MA3, False, F64),
+    case(Q19, (82, 81, 64), GUO, F.Constant, MA3, True, F64),
+    case(Q27, (57, 255, 129), NONE, F.None_, MA3, False, F64),
 ]
 
 
 def kernel_of(c):
-    """(kernel index, limit) of tests/native/march_rules.cpp."""
+    """Columns, interior columns, force table entries, values to a line and cost limit
+    of the two-step kernel."""
     q27, exact = c["lattice"] == Q27, c["equilibrium"] == EXACT
-    source = c["scheme"] != NONE
-    side = source and c["force"] in (F.Kolmogorov, F.Sinusoidal)
-    limit = 3.9 if exact and source else 6.1 if q27 else 5.3 if c["scheme"] == EDM else 13.0
-    return 2 * q27 + side, limit
+    source, fp64 = c["scheme"] != NONE, c["numbers"] == F64
+    side = 264 if source and c["force"] in (F.Kolmogorov, F.Sinusoidal) else 0
+    limit = (4.9 if fp64 else 3.9 if exact and source else 6.1 if q27 else
+             5.3 if c["scheme"] == EDM else 13.0)
+    size = 8 if fp64 else 4
+    lds = 163840 - 3 * side * size
+    interior = 512 if fp64 else 1024 if q27 else 2048
+    return lds // ((24 if q27 else 16) * size) // 4 * 4, interior, side, 128 // size, limit

@@ -14,16 +14,19 @@ static void check(bool ok, const char* what, int nx, int ny, int nz, int columns
   ++failures;
 }
 
-// (columns, interior, side) of D3Q19 and D3Q27 in FP32, without and with force tables
-static const int kernels[4][3] = {
-    {2560, 2048, 0}, {2510, 2048, 264}, {1704, 1024, 0}, {1672, 1024, 264}};
+// (columns, interior, side) of D3Q19 and D3Q27 in FP32 and in FP64, without and with
+// force tables
+static const int kernels[8][3] = {
+    {2560, 2048, 0}, {2508, 2048, 264}, {1704, 1024, 0}, {1672, 1024, 264},
+    {1280, 512, 0},  {1228, 512, 264},  {852, 512, 0},   {820, 512, 264}};
 
 int main(int argc, char** argv) {
-  if (argc == 6) {  // nx ny nz kernel limit
-    const int* k = kernels[std::atoi(argv[4])];
-    const int nx = std::atoi(argv[1]), ny = std::atoi(argv[2]), nz = std::atoi(argv[3]);
-    const lbm::MarchShape m = lbm::march_shape(nx, ny, nz, k[0], k[1], k[2], 256, 32);
-    std::printf("%d\n", (int)lbm::march_pays(m, (double)nx * ny * nz, k[1], std::atof(argv[5])));
+  if (argc == 9) {  // nx ny nz columns interior side line limit
+    int v[8];
+    for (int k = 1; k < 8; ++k) v[k] = std::atoi(argv[k]);
+    const lbm::MarchShape m = lbm::march_shape(v[1], v[2], v[3], v[4], v[5], v[6], 256, v[7]);
+    std::printf("%d\n", (int)lbm::march_pays(m, (double)v[1] * v[2] * v[3], v[5],
+                                             std::atof(argv[8])));
     return 0;
   }
   const int extents[] = {1,   2,   3,   7,    8,    9,    31,   32,   33,    64,     96,

@@ -1,6 +1,7 @@
 """The two-step kernel against the one-cell-per-lane kernel.
 
-Tolerance: a step rounds each population to FP32 after sums of at most 27 terms
+FP64 arithmetic: the same bits (separately rounded operations in the same order).
+Tolerance in FP32: a step rounds each population to FP32 after sums of at most 27 terms
 on either side, so two correct kernels differ by at most 2 x 30 x 2^-24 of the
 largest population a step, and BGK at tau > 1/2 near equilibrium does not amplify
 it; a misplaced population is off by the noise, 1e-2 of the weights."""
@@ -10,8 +11,8 @@ import os
 import numpy as np
 import pytest
 
-from march_cases import CASES
-from metalbm_amd import Algorithm, Config, KernelShape, Precision
+from march_cases import CASES, F64
+from metalbm_amd import Algorithm, Config, KernelShape
 
 pytestmark = pytest.mark.gpu
 ULP = 2 * 30 * 2.0 ** -24
@@ -22,13 +23,14 @@ def config(c, kernel=KernelShape.AUTO):
     return Config(lattice=c["lattice"], nx=n[0], ny=n[1], nz=n[2], tau=0.55,
                   forcing_scheme=c["scheme"], force=c["force"], equilibrium=c["equilibrium"],
                   amplitude=(1e-5, 2e-5, -1e-5), wavelength=(n[1] / 3, 17.0, 9.0),
-                  storage=Precision.F32, compute=Precision.F32, shifted=c["shifted"],
+                  storage=c["numbers"][0], compute=c["numbers"][1], shifted=c["shifted"],
                   kernel=kernel)
 
 
 def name(c):
     return (f"{c['lattice'].name}-{'x'.join(map(str, c['shape']))}-{c['scheme'].name}-"
-            f"{c['force'].name}-{c['equilibrium'].name}-{'shifted' if c['shifted'] else 'plain'}")
+            f"{c['force'].name}-{c['equilibrium'].name}-{'shifted' if c['shifted'] else 'plain'}-"
+            f"{c['numbers'][0].name}-{c['numbers'][1].name}")
 
 
 def noisy(a):
@@ -46,6 +48,8 @@ def test_two_steps_per_launch(c):
             out.append((a.populations(), a.reduce()))
             assert a.steps_done == steps
     scale = np.abs(out[1][0]).max()
+    if c["numbers"] == F64:
+        assert np.array_equal(out[0][0], out[1][0])
     assert np.abs(out[0][0] - out[1][0]).max() <= steps * ULP * scale
     assert out[0][1][0] == pytest.approx(out[1][1][0], rel=steps * ULP)
 

@@ -23,7 +23,6 @@ def test_tiling(tmp_path):
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout
     for c in CASES:
-        kernel, limit = kernel_of(c)
-        r = subprocess.run([exe, *map(str, c["shape"]), str(kernel), str(limit)],
-                           capture_output=True, text=True, timeout=60)
+        r = subprocess.run([exe, *map(str, c["shape"] + kernel_of(c))], capture_output=True,
+                           text=True, timeout=60)
         assert r.stdout.strip() == "1", c
