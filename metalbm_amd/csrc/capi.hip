@@ -64,6 +64,8 @@ struct lbm_handle {
   StepFn step = nullptr;
   MarchFn march = nullptr;  // two steps in one launch (NULL: one step at a time)
   MarchTiling tiling{};
+  TileFn tile = nullptr;  // 2D: up to tile2d.steps steps in one launch (NULL: one)
+  Tile2D tile2d{};
   int64_t steps = 0;
   double w[27], scale[27];
   std::string err;
@@ -175,6 +177,28 @@ void choose_march(lbm_handle* h) {
   if (!march_pays(m, (double)h->N, k.interior, limit)) return;
   h->march = k.launch[side];
   h->tiling = MarchTiling{m.ty, m.tz, m.tiles_y, m.tiles_z, m.ranges};
+}
+
+// The multi-step kernel of a 2D domain, under the same condition.
+void choose_tile(lbm_handle* h) {
+  const lbm_config& c = h->cfg;
+  if (c.collision != LBM_BGK || c.kernel != LBM_KERNEL_AUTO || h->D != 2) return;
+  const KernelKey key{c.lattice, c.collision, src_of(c.forcing_scheme), c.equilibrium,
+                      c.storage, h->ctype, c.shifted ? 1 : 0};
+  const TileKernel k = registry().find_tile(key);
+  // byte offsets within a population are 32-bit
+  if (!k.launch[0] || (double)h->N * (double)h->elem >= 4294967296.0) return;
+  const TileShape shape =
+      tile_shape(c.nx, c.ny, k.rows, h->ctype == TYPE_F64, c.equilibrium == LBM_EQ_EXACT);
+  if (shape.steps < 2) return;
+  Tile2D m{};
+  m.steps = shape.steps;
+  m.tx = shape.tx;
+  m.ty = shape.ty;
+  m.tiles_x = (c.nx + m.tx - 1) / m.tx;
+  m.tiles_y = (c.ny + m.ty - 1) / m.ty;
+  h->tile = k.launch[shape.wide];
+  h->tile2d = m;
 }
 
 // Force tables (Force.h:154-159, 208-215, 262-267), FP64 on the host with the
@@ -595,6 +619,7 @@ int lbm_create(const lbm_config* cfg, lbm_handle** out) {
   h->own_stream = true;
   if (int rc = build_force_tables(h)) return bail(rc);
   choose_march(h);
+  choose_tile(h);
   if (cfg->collision == LBM_ELBM) {
     const size_t ab = (size_t)h->N * (h->ctype == TYPE_F64 ? 8 : 4);
     e = hipMalloc(&h->alpha, ab);
@@ -945,7 +970,21 @@ int lbm_step(lbm_handle* h, int nsteps, int store_last) {
   // caller that keeps lbm_device_populations across them), and never the storing
   // step.
   int paired = h->march ? (nsteps - (store_last ? 1 : 0)) / 4 * 4 : 0;
-  for (int s = 0; s < nsteps; ++s) {
+  // The 2D kernel stores as well; as many launches, modulo two, as steps.
+  int launches = nsteps;
+  if (h->tile && nsteps > 1) {
+    launches = (nsteps + h->tile2d.steps - 1) / h->tile2d.steps;
+    launches += (nsteps - launches) & 1;
+  }
+  for (int s = 0, n = 1; s < nsteps; s += n) {
+    if (paired > 0) {
+      n = 2;
+      paired -= 2;
+    } else if (h->tile) {
+      n = (nsteps - s + launches - 1) / launches--;
+    } else {
+      n = 1;
+    }
     // Collision::update before the step (Algorithm.h:338, Collision.h:96-99);
     // ConstantShell is set once (Collision.h:51-54).  EnergyRemoval and
     // Turbulent2D read only the fields of the last storing step, which change
@@ -959,7 +998,7 @@ int lbm_step(lbm_handle* h, int nsteps, int store_last) {
     }
     a.src = h->f[h->cur];
     a.dst = h->f[1 - h->cur];
-    a.store = (store_last && s == nsteps - 1) ? 1 : 0;
+    a.store = (store_last && s + n == nsteps) ? 1 : 0;
     if (a.defer.cells) {
       a.defer.count = h->defer_count + (s & 1) * kDeferCounters;
       a.defer.next = h->defer_count + (1 - (s & 1)) * kDeferCounters;
@@ -971,19 +1010,19 @@ int lbm_step(lbm_handle* h, int nsteps, int store_last) {
       a.alpha_out = h->fields + (size_t)h->N * (1 + h->D);
       a.F_out = h->fields + (size_t)h->N * (2 + h->D);
     }
-    if (paired > 0) {
-      const hipError_t e = h->march(a, h->tiling, h->stream);
-      if (e != hipSuccess) return hip_fail(h, e, "two-step launch");
-      h->cur = 1 - h->cur;
-      h->steps += 2;
-      paired -= 2;
-      ++s;
-      continue;
+    hipError_t e;
+    if (n == 1) {
+      e = h->step(a, h->cfg.forcing_scheme, h->block, grid, h->stream);
+    } else if (h->tile) {
+      Tile2D m = h->tile2d;
+      m.steps = n;
+      e = h->tile(a, m, h->cfg.forcing_scheme, h->stream);
+    } else {
+      e = h->march(a, h->tiling, h->stream);
     }
-    hipError_t e = h->step(a, h->cfg.forcing_scheme, h->block, grid, h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "fused step launch");
     h->cur = 1 - h->cur;
-    h->steps += 1;
+    h->steps += n;
   }
   if (store_last) {
     h->fields_valid = true;

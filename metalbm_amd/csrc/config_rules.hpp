@@ -246,4 +246,63 @@ inline bool march_pays(const MarchShape& m, double cells, int interior, double l
   return m.ranges > 0 && cells >= 262144.0 && 2 * m.ty * m.tz >= interior && m.cost <= limit;
 }
 
+// Tiling of the multi-step 2D kernel: rows of 16 cells (wide 0) or of 64 with the
+// halo, tx x ty cells without it, up to `steps` steps in a launch (0: one step at a
+// time is faster).  rows: rows of each width that a workgroup holds.  From 14 sizes
+// from 32^2 to 2048^2 (a launch costs 2.5 us, a step 4.1 to 4.9 us with it on the
+// small ones), five steps to a launch were the best of 3, 4, 5 and 7; time over the
+// one-step kernel's, Ma3 with the Guo source in FP64 / FP32 / FP16, then the product
+// equilibrium with the exact-difference source:
+//   16-cell rows, 8 x 8 tiles, up to 256 of them (128^2: 0.46 / 0.32 / 0.34, 0.44 to
+//   0.49), taller ones up to 24 x 8 (192^2: 0.57 / 0.36 / 0.37, 0.58 to 0.60); at 256^2
+//   64-cell rows are the better ones (0.68 / 0.43 / 0.44 against 0.79 / 0.44 / 0.48);
+//   64-cell rows: the tile whose row passes (eight wavefronts, 512 workgroups at once,
+//   the rows shrinking with the steps) and launches cost least per step: 320^2, 8 rows:
+//   0.56 / 0.41 / 0.40; 512^2, 16 rows: 0.81 / 0.55 / 0.78; 2048^2, all rows: 0.72 /
+//   0.42 / 0.61, in FP64 with three steps (five: 0.79).  On domains of more than 512
+//   tiles of 8 rows the product equilibrium gains in FP64 only (0.58 to 0.92; FP32
+//   0.76 to 1.15, FP16 1.0 to 1.3).
+// Tiles narrower than half a row leave lanes idle.
+struct TileShape {
+  int wide = 0, steps = 0, tx = 0, ty = 0;
+};
+inline TileShape tile_shape(int nx, int ny, const int (&rows)[2], bool fp64, bool exact) {
+  auto fit = [&](int wide, int steps, int tx) {
+    TileShape m;
+    const int halo = steps - 1, width = wide ? 64 : 16;
+    m.wide = wide;
+    m.ty = ny <= width ? ny : width - 2 * halo;
+    m.tx = tx >= nx || halo > nx ? nx : tx;
+    if (m.tx + (m.tx == nx ? 0 : 2 * halo) <= rows[wide] && 2 * m.ty >= width - 2 * halo)
+      m.steps = steps;
+    return m;
+  };
+  auto groups = [&](const TileShape& m) {
+    return (long long)((nx + m.tx - 1) / m.tx) * ((ny + m.ty - 1) / m.ty);
+  };
+  if ((long long)nx * ny <= 49152)
+    for (int tx : {8, 16, 24}) {
+      const TileShape m = fit(0, 5, tx);
+      if (m.steps && groups(m) <= 256) return m;
+    }
+  if (exact && !fp64 && groups(fit(1, 5, 8)) > 512) return TileShape{};
+  TileShape best;
+  double least = 0.0;
+  for (int steps = 5; steps >= (fp64 ? 3 : 5); steps -= 2)
+    for (int tx : {8, 16, 24, 32, rows[1] - 2 * (steps - 1)}) {
+      const TileShape m = fit(1, steps, tx);
+      if (!m.steps) continue;
+      int passes = 0;
+      for (int t = 1; t <= steps; ++t)
+        passes += (m.tx + (m.tx == nx ? 0 : 2 * (steps - t)) + 7) / 8;
+      // a launch takes as long as 2.5 row passes in FP64, 5 in FP32
+      const double cost =
+          ((double)((groups(m) + 511) / 512) * passes + (fp64 ? 2.5 : 5.0)) / steps;
+      if (best.steps && cost >= least) continue;
+      best = m;
+      least = cost;
+    }
+  return best;
+}
+
 }  // namespace lbm

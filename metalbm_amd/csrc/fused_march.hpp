@@ -65,19 +65,6 @@ constexpr int march_slot() {
   return k;
 }
 
-template <class L, class C, int FS, int EQ, bool SH, class EMIT>
-__device__ __forceinline__ void march_collide(const StepArgs& a, const C* f, const C* F, C& rho,
-                                              C* u, EMIT&& emit) {
-  if constexpr (std::is_same_v<C, float> && EQ == (int)EquilibriumType::TruncationMa3)
-    bgk_collide_pairs<L, FS, SH>(a, f, F, rho, u, emit);
-  else
-    bgk_collide<L, C, FS, EQ, SH>(a, f, F, rho, u, emit);
-}
-
-__device__ __forceinline__ int wrap_index(int v, int n) {
-  return v < 0 ? v + n : (v >= n ? v - n : v);
-}
-
 // SIDE: forces that vary along y or z.
 template <class L, class S, class C, int FS, int EQ, bool SH, bool SIDE>
 __global__ void __launch_bounds__(kMarchThreads)
@@ -206,7 +193,7 @@ __global__ void __launch_bounds__(kMarchThreads)
         h[i] = to_compute<L, i, S, C>(p[i]);
       });
       force_at(c, xs, F);
-      march_collide<L, C, FS, EQ, SH>(a, h, F, rho, u, [&](auto ic, C v) {
+      bgk_collide_fast<L, C, FS, EQ, SH>(a, h, F, rho, u, [&](auto ic, C v) {
         constexpr int i = decltype(ic)::value, slot = march_slot<L, i>();
         const S s = to_storage<L, i, S, C>(v);
         if constexpr (slot >= 0) {
@@ -268,7 +255,7 @@ __global__ void __launch_bounds__(kMarchThreads)
         force_at(c, xd, F);
         const unsigned cell = (unsigned)((y0 + row_of(c) - 1) * a.nz + (z0 + z - rim_z)) *
                               (unsigned)sizeof(S);
-        march_collide<L, C, FS, EQ, SH>(a, h, F, rho, u, [&](auto ic, C v) {
+        bgk_collide_fast<L, C, FS, EQ, SH>(a, h, F, rho, u, [&](auto ic, C v) {
           constexpr int i = decltype(ic)::value;
           char* base = reinterpret_cast<char*>(dst + (size_t)i * (size_t)a.N + (size_t)xd * plane);
           store_pop<L, i, S, C>(reinterpret_cast<S*>(base + cell), v);

@@ -223,6 +223,16 @@ __device__ __forceinline__ void bgk_collide(const StepArgs& a, const C* f, const
   }
 }
 
+// The form that the kernels of several steps take.
+template <class L, class C, int FS, int EQ, bool SH, class EMIT>
+__device__ __forceinline__ void bgk_collide_fast(const StepArgs& a, const C* f, const C* F, C& rho,
+                                              C* u, EMIT&& emit) {
+  if constexpr (std::is_same_v<C, float> && EQ == (int)EquilibriumType::TruncationMa3)
+    bgk_collide_pairs<L, FS, SH>(a, f, F, rho, u, emit);
+  else
+    bgk_collide<L, C, FS, EQ, SH>(a, f, F, rho, u, emit);
+}
+
 // FSX: the forcing scheme as configured (None vs Shan-Chen matters only for
 // the stored hydrodynamic velocity), passed at run time.
 // NT: non-temporal population loads (chosen per configuration by the host).

@@ -9,6 +9,7 @@
 #include "fused_march.hpp"
 #include "fused_step.hpp"
 #include "fused_step_vec.hpp"
+#include "fused_tile.hpp"
 #include "registry.hpp"
 
 namespace lbm {
@@ -101,6 +102,13 @@ MarchKernel march_kernel() {
   return k;
 }
 
+template <class L, class S, class C, int FS, int EQ, bool SH, int W>
+hipError_t launch_tile(const StepArgs& a, const Tile2D& m, int fsx, hipStream_t st) {
+  hipLaunchKernelGGL((k_bgk_tile<L, S, C, FS, EQ, SH, W>), dim3(m.tiles_x * m.tiles_y),
+                     dim3(kTileThreads), 0, st, a, m, fsx);
+  return hipGetLastError();
+}
+
 template <class L, class S, class C, bool SH, int... Vs>
 void register_combo(Registry& r, int storage, int compute) {
   auto add_eq = [&](auto eqc) {
@@ -117,6 +125,11 @@ void register_combo(Registry& r, int storage, int compute) {
       if constexpr (L::dimD == 3 && std::is_same_v<S, C> && !HEAVY)
         r.add({(int)L::Type, (int)CollisionType::BGK, FS, EQ, storage, compute, SH, 0},
               march_kernel<L, S, C, FS, EQ, SH>());
+      if constexpr (L::dimD == 2 && sizeof(S) <= sizeof(C))
+        r.add({(int)L::Type, (int)CollisionType::BGK, FS, EQ, storage, compute, SH, 0},
+              TileKernel{{&launch_tile<L, S, C, FS, EQ, SH, 16>,
+                          &launch_tile<L, S, C, FS, EQ, SH, 64>},
+                         {kTileRows<L, S, 16>, kTileRows<L, S, 64>}});
       r.add({(int)L::Type, (int)CollisionType::ELBM, FS, EQ, storage, compute, SH, 0},
             &launch_step<L, S, C, FS, EQ, SH, (int)CollisionType::ELBM>);
       (r.add({(int)L::Type, (int)CollisionType::BGK, FS, EQ, storage, compute, SH, Vs},

@@ -29,6 +29,14 @@ struct MarchKernel {
   int interior = 0, side = 0;
 };
 
+// The multi-step kernel of a 2D configuration, for tiles in rows of 16 and of 64 cells,
+// and the rows that a workgroup holds.
+using TileFn = hipError_t (*)(const StepArgs&, const Tile2D&, int fsx, hipStream_t);
+struct TileKernel {
+  TileFn launch[2] = {nullptr, nullptr};
+  int rows[2] = {0, 0};
+};
+
 // vec = 0 selects the one-cell-per-lane kernel; vec = V > 0 the kernel in
 // which each lane owns V consecutive cells (aligned vector accesses).
 struct KernelKey {
@@ -46,6 +54,12 @@ struct Registry {
   MarchKernel find_march(const KernelKey& k) const {
     auto it = march.find(k.code());
     return it == march.end() ? MarchKernel{} : it->second;
+  }
+  std::map<int64_t, TileKernel> tile;
+  void add(const KernelKey& k, const TileKernel& f) { tile[k.code()] = f; }
+  TileKernel find_tile(const KernelKey& k) const {
+    auto it = tile.find(k.code());
+    return it == tile.end() ? TileKernel{} : it->second;
   }
   void add(const KernelKey& k, StepFn f) { step[k.code()] = f; }
   StepFn find(const KernelKey& k) const {

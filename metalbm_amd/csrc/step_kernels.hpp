@@ -104,6 +104,12 @@ struct MarchTiling {
   int ty, tz, tiles_y, tiles_z, ranges;
 };
 
+// Tiling of the multi-step 2D kernel (fused_tile.hpp): tiles of tx x ty cells, steps
+// in one launch.
+struct Tile2D {
+  int tx, ty, tiles_x, tiles_y, steps;
+};
+
 // Storage / compute codes (values of LBM_F64 / LBM_F32 / LBM_F16).
 enum : int { TYPE_F64 = 0, TYPE_F32 = 1, TYPE_F16 = 2 };
 
@@ -163,6 +169,10 @@ struct CellPos {
   int x, y, z, xm, xp, ym, yp, zm, zp;
   bool active;
 };
+
+__device__ __forceinline__ int wrap_index(int v, int n) {
+  return v < 0 ? v + n : (v >= n ? v - n : v);
+}
 
 template <class L, int BLOCK>
 __device__ __forceinline__ CellPos cell_of_thread(const StepArgs& a) {
