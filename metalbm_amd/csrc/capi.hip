@@ -7,11 +7,13 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/metalbm_amd.h"
@@ -40,6 +42,10 @@ const Registry& registry() {
 }
 }  // namespace lbm
 
+// Pinned chunks, two to a copying thread.
+constexpr int kRingSlots = 8;
+constexpr size_t kRingChunk = 1 << 20;
+
 struct lbm_handle {
   lbm_config cfg{};
   int device = 0;           // the HIP device current at lbm_create
@@ -56,6 +62,8 @@ struct lbm_handle {
   uint64_t fields_version = 0;  // bumped whenever the fields are rewritten
   double* staging = nullptr;   // N doubles
   double* reduce_buf = nullptr;
+  char* ring = nullptr;     // pinned chunks of lbm_get_fields, and their events
+  hipEvent_t ring_event[kRingSlots] = {};
   void* ftab[3] = {nullptr, nullptr, nullptr};
   int fax[3] = {3, 3, 3};
   unsigned long long* stats = nullptr;  // kStatSlots x kStatStride counters
@@ -296,6 +304,92 @@ int ensure_fields(lbm_handle* h) {
   return LBM_OK;
 }
 
+// Fields to pageable host memory.  Left to the runtime, one thread fills the caller's
+// pages, most of them touched for the first time: 12 GB/s of the link's 54.  Here the
+// chunks go to pinned memory and four threads empty it, each with one chunk on its
+// way while it copies the other (35 MB, ten steps of D3Q19 96 x 80 x 72 and the copy:
+// 3.41 -> 1.70 ms; 94 MB: 9.8 -> 4.1; 12 MB: 0.90 -> 0.63).  Requests of fewer bytes
+// than the pinned memory, and pinned or device destinations, are copied directly.
+struct FieldPart {
+  char* dst;
+  const char* src;
+  size_t bytes;
+};
+bool ensure_ring(lbm_handle* h) {
+  if (h->ring) return true;
+  char* mem = nullptr;
+  bool ok = hipHostMalloc(&mem, kRingSlots * kRingChunk, hipHostMallocDefault) == hipSuccess;
+  for (int k = 0; ok && k < kRingSlots; ++k)
+    if (!h->ring_event[k])
+      ok = hipEventCreateWithFlags(&h->ring_event[k], hipEventDisableTiming) == hipSuccess;
+  if (ok) {
+    h->ring = mem;
+  } else {
+    (void)hipGetLastError();
+    if (mem) (void)hipHostFree(mem);
+  }
+  return ok;
+}
+bool pageable(const void* p) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();  // memory that HIP does not know
+  return true;
+}
+hipError_t copy_through_ring(lbm_handle* h, const FieldPart* parts, int n_parts) {
+  std::atomic<size_t> next{0};
+  std::atomic<int> error{hipSuccess};
+  auto chunk = [&](size_t k, FieldPart* c) {
+    for (int p = 0; p < n_parts; ++p) {
+      const size_t chunks = (parts[p].bytes + kRingChunk - 1) / kRingChunk;
+      if (k < chunks) {
+        const size_t at = k * kRingChunk;
+        *c = {parts[p].dst + at, parts[p].src + at, std::min(kRingChunk, parts[p].bytes - at)};
+        return true;
+      }
+      k -= chunks;
+    }
+    return false;
+  };
+  auto work = [&](int w) {
+    FieldPart c[2];
+    auto issue = [&](int k) {
+      if (error != hipSuccess || !chunk(next++, &c[k])) return false;
+      const int slot = 2 * w + k;
+      hipError_t e = hipMemcpyAsync(h->ring + slot * kRingChunk, c[k].src, c[k].bytes,
+                                    hipMemcpyDeviceToHost, h->stream);
+      if (e == hipSuccess) e = hipEventRecord(h->ring_event[slot], h->stream);
+      if (e != hipSuccess) error = e;
+      return e == hipSuccess;
+    };
+    if (w > 0 && hipSetDevice(h->device) != hipSuccess) return;
+    bool have = issue(0);
+    for (int k = 0; have; k ^= 1) {
+      have = issue(k ^ 1);
+      const int slot = 2 * w + k;
+      const hipError_t e = hipEventSynchronize(h->ring_event[slot]);
+      if (e != hipSuccess) {
+        error = e;
+        break;
+      }
+      std::memcpy(c[k].dst, h->ring + slot * kRingChunk, c[k].bytes);
+    }
+  };
+  std::thread helpers[kRingSlots / 2];
+  for (int w = 1; w < kRingSlots / 2; ++w) {
+    try {
+      helpers[w] = std::thread(work, w);
+    } catch (...) {  // no thread to be had: the others copy its share
+      break;
+    }
+  }
+  work(0);
+  for (auto& t : helpers)
+    if (t.joinable()) t.join();
+  const hipError_t e = hipStreamSynchronize(h->stream);
+  return error != hipSuccess ? (hipError_t)error.load() : e;
+}
+
 // State every initialiser starts from.  The entropic alpha field restarts at
 // 2 (initAlpha, Initialize.h:81-88), so a re-initialised handle matches a
 // fresh one.  The reference's field list holds the initial density and
@@ -321,6 +415,9 @@ hipError_t seed_state(lbm_handle* h, const double* drho, double rho0, const doub
 }
 
 void release(lbm_handle* h) {
+  if (h->ring) (void)hipHostFree(h->ring);
+  for (hipEvent_t e : h->ring_event)
+    if (e) (void)hipEventDestroy(e);
   lbm::release_spectral(h->spectral);
   h->spectral = nullptr;
   if (h->ffield) {  // ftab points into the force field
@@ -1037,17 +1134,33 @@ int lbm_get_fields(lbm_handle* h, double* rho, double* u_hydro, double* alpha,
   if (!h->fields_valid)
     return fail(h, LBM_E_STATE, "no storing step has run (lbm_step store_last)");
   const size_t n = (size_t)h->N;
-  struct {
-    double* dst;
-    size_t off, count;
-  } parts[4] = {{rho, 0, n},
-                {u_hydro, n, n * h->D},
-                {alpha, n * (1 + h->D), n},
-                {force, n * (2 + h->D), n * h->D}};
-  for (auto& p : parts)
-    if (p.dst)
-      HIP_TRY(h, hipMemcpyAsync(p.dst, h->fields + p.off, p.count * sizeof(double),
-                                hipMemcpyDeviceToHost, h->stream));
+  double* const dst[4] = {rho, u_hydro, alpha, force};
+  const size_t off[5] = {0, n, n * (1 + h->D), n * (2 + h->D), n * (2 + 2 * h->D)};
+  FieldPart parts[4];
+  int n_parts = 0;
+  size_t bytes = 0;
+  bool plain = true;
+  for (int k = 0; k < 4; ++k) {
+    if (!dst[k]) continue;
+    parts[n_parts] = {reinterpret_cast<char*>(dst[k]),
+                      reinterpret_cast<const char*>(h->fields + off[k]),
+                      (off[k + 1] - off[k]) * sizeof(double)};
+    bytes += parts[n_parts++].bytes;
+    plain = plain && pageable(dst[k]);
+  }
+  if (plain && bytes >= kRingSlots * kRingChunk) {
+    int current = -1;
+    HIP_TRY(h, hipGetDevice(&current));
+    if (current != h->device) HIP_TRY(h, hipSetDevice(h->device));
+    const bool ring = ensure_ring(h);
+    const hipError_t e = ring ? copy_through_ring(h, parts, n_parts) : hipSuccess;
+    if (current != h->device) (void)hipSetDevice(current);
+    HIP_TRY(h, e);
+    if (ring) return LBM_OK;
+  }
+  for (int k = 0; k < n_parts; ++k)
+    HIP_TRY(h, hipMemcpyAsync(parts[k].dst, parts[k].src, parts[k].bytes, hipMemcpyDeviceToHost,
+                              h->stream));
   HIP_TRY(h, hipStreamSynchronize(h->stream));
   return LBM_OK;
 }
