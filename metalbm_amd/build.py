@@ -29,6 +29,7 @@ COMMON = ["-O3", f"--offload-arch={ARCH}", "-std=c++17", "-fPIC",
           "-Wno-unused-command-line-argument", f"-I{INCLUDE}"]
 SOURCES = {
     "step_f32_d3q27.hip": ["-ffp-contract=fast"],
+    "step_mixed_d3q27.hip": ["-ffp-contract=fast"],
     "step_f32_d3q19.hip": ["-ffp-contract=fast"],
     "step_f32_d2q9.hip": ["-ffp-contract=fast"],
     "step_f64_d3q27.hip": ["-ffp-contract=off"],

@@ -36,6 +36,7 @@ const Registry& registry() {
     register_step_f32_d2q9(x);
     register_step_f32_d3q19(x);
     register_step_f32_d3q27(x);
+    register_step_mixed_d3q27(x);
     return x;
   }();
   return r;

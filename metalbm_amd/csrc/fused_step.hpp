@@ -555,8 +555,8 @@ __device__ __forceinline__ unsigned sample_hash(unsigned cell, unsigned salt) {
 // step), and 45 us in dense wavefronts of their own.
 //
 // Measured per step, term by term for every cell -> power sums and list:
-// reference Newton D2Q9 2048^2 474 -> 206 us, D3Q27 256^3 5.75 -> 1.77 ms; plain
-// Newton D3Q27 4.83 -> 1.76 ms, stored-alpha correction D3Q27 4.23 -> 1.78 ms.
+// reference Newton D2Q9 2048^2 474 -> 190 us, D3Q27 256^3 5.75 -> 1.70 ms; plain
+// Newton D3Q27 4.83 -> 1.65 ms, stored-alpha correction D3Q27 4.23 -> 1.70 ms.
 // D2Q9's other modes take one or two evaluations in the log1p form already,
 // most of what the power sums cost (147-167 us of 153), and stay.
 // Three phases so that the learned mode's wavefront-wide matrix-core

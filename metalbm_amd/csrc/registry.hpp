@@ -74,6 +74,7 @@ void register_step_f64_d3q27(Registry& r);
 void register_step_f32_d2q9(Registry& r);
 void register_step_f32_d3q19(Registry& r);
 void register_step_f32_d3q27(Registry& r);
+void register_step_mixed_d3q27(Registry& r);
 
 const Registry& registry();
 
