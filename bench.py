@@ -2,12 +2,14 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME]
 
-Prints ONE JSON line on stdout.  A step is one fused kernel launch over the
+Prints ONE JSON line on stdout.  A step is one collide-and-stream over the
 whole lattice (inputs resident in HBM).  `value` is MLUPS = cells * K / t
 (wall clock of the K timed steps, device synchronised on both sides).  The
-roofline block divides the algorithmic bytes per launch (2 Q sizeof(storage)
-per cell, plus the alpha state for Newton ELBM) by the average kernel
-duration measured with HIP events on the stream the kernels run on.  The CPU
+roofline block divides the algorithmic bytes of a step (2 Q sizeof(storage)
+per cell, plus the alpha state for Newton ELBM) by the average time of a step
+measured with HIP events on the stream the kernels run on.  Kernels that take
+several steps in one pass over the lattice move fewer bytes than that, so the
+rate counted this way can exceed the peak; `traffic` is what a step moves.  The CPU
 baseline is the FP64 oracle (a restatement of the reference's CPU loop,
 OpenMP over x) timed on a bounded sample of the same workload on this host.
 """
@@ -681,6 +683,7 @@ def stream_ceiling(K: int, W: int, name: str = DEFAULT) -> dict:
     if wl["cfg"].get("collision", "BGK") != "BGK":
         raise SystemExit("--stream-ceiling takes a BGK workload")
     cfg = make_config(wl["cfg"])
+    cfg.kernel = m.kernel_shape(cfg)[0]  # one step a launch, as the probes' pattern
     hip = Hip()
     a = m.Algorithm(cfg)
     s = hip.stream()
@@ -701,7 +704,7 @@ def stream_ceiling(K: int, W: int, name: str = DEFAULT) -> dict:
     out = {"metric": "achieved HBM bandwidth of the step kernel vs probes of its access pattern",
            "unit": "GB/s", "steps": K, "warmup": W,
            "config": {"workload": name, "cells": N, "bytes_per_population": pop,
-                      "step_kernel": m.kernel_shape(cfg)[0].name.lower()}}
+                      "step_kernel": cfg.kernel.name.lower()}}
     ms = timed(lambda k: a.iterate(k))
     out["step"] = {"us": round(ms * 1e3, 2), "bytes": 2 * Q * pop,
                    "GB/s": round(2 * Q * pop / ms / 1e6, 1)}
@@ -719,7 +722,7 @@ def stream_ceiling(K: int, W: int, name: str = DEFAULT) -> dict:
 
 
 def traffic_of(name):
-    """HBM bytes per launch of the workload's step kernel, from the committed
+    """HBM bytes per step of the workload's step kernel, from the committed
     rocprofv3 FETCH_SIZE / WRITE_SIZE summary (profiles/traffic_<name>.txt,
     counters scaled by a copy of known size), or None when not measured."""
     p = os.path.join(ROOT, "profiles", f"traffic_{name}.txt")
@@ -727,7 +730,7 @@ def traffic_of(name):
         return None
     with open(p) as fh:
         for line in fh:
-            if line.startswith("hbm_bytes_per_launch:"):
+            if line.startswith("hbm_bytes_per_step:"):
                 return int(line.split(":", 1)[1])
     return None
 
