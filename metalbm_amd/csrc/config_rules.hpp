@@ -261,7 +261,8 @@ inline bool march_pays(const MarchShape& m, double cells, int interior, double l
 //   0.56 / 0.41 / 0.40; 512^2, 16 rows: 0.81 / 0.55 / 0.78; 2048^2, all rows: 0.72 /
 //   0.42 / 0.61, in FP64 with three steps (five: 0.79).  On domains of more than 512
 //   tiles of 8 rows the product equilibrium gains in FP64 only (0.58 to 0.92; FP32
-//   0.76 to 1.15, FP16 1.0 to 1.3).
+//   0.76 to 1.15, FP16 1.0 to 1.3).  (FP16 without its conversions' products takes
+//   another 2 to 12 % less with Ma3.)
 // Tiles narrower than half a row leave lanes idle.
 struct TileShape {
   int wide = 0, steps = 0, tx = 0, ty = 0;

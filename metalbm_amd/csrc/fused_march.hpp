@@ -33,10 +33,11 @@
 // the vector issue slots), D3Q27 193 x 161 x 130 Ma3 260 -> 159, product
 // equilibrium 276 -> 183; FP64, one column a thread: D3Q19 192^3 424 -> 328, 171 x
 // 150 x 133 257 -> 208 (60 % of the issue slots: before opposite populations shared
-// their terms 246, with divisions by 6 and 24 304).  FP16 (1245 against 1211 at D3Q27
-// 384^3: as many vector instructions for half the bytes) stays with the one-step
-// kernels, and so does FP64 storage with FP32 arithmetic, whose populations would
-// show that the two kernels round their FP32 sums differently.
+// their terms 246, with divisions by 6 and 24 304).  FP16 (D3Q27 384^3, waiting
+// populations packed in pairs: 1162 against 1205, 72 % of the issue slots at half the
+// bytes, but 192^3 1.01 to 1.21 and 64^3 2.2 times the one-step kernel's time) stays
+// with the one-step kernels, and so does FP64 storage with FP32 arithmetic, whose
+// populations would show that the two kernels round their FP32 sums differently.
 #pragma once
 
 #include "fused_step.hpp"
@@ -186,16 +187,11 @@ __global__ void __launch_bounds__(kMarchThreads)
     const int xs = wrap_index(x, a.nx);
     S mine[U][3];  // the populations that stay in their column, by c_x + 1
     auto step_one = [&](int c, const S (&p)[Q], auto&& stays) {
-      C h[Q], F[3], rho, u[3];
+      C F[3], rho, u[3];
       S* const to = lds + (row_of(c) * pitch + place_of(c));
-      static_for<Q>([&](auto ic) {
-        constexpr int i = decltype(ic)::value;
-        h[i] = to_compute<L, i, S, C>(p[i]);
-      });
       force_at(c, xs, F);
-      bgk_collide_fast<L, C, FS, EQ, SH>(a, h, F, rho, u, [&](auto ic, C v) {
+      bgk_collide_stored<L, S, C, FS, EQ, SH>(a, p, F, rho, u, [&](auto ic, S s) {
         constexpr int i = decltype(ic)::value, slot = march_slot<L, i>();
-        const S s = to_storage<L, i, S, C>(v);
         if constexpr (slot >= 0) {
           if (c >= 0) to[slot * COLUMNS] = s;
         } else {
@@ -247,18 +243,19 @@ __global__ void __launch_bounds__(kMarchThreads)
       if (x > x0 && c >= 0) {
         // plane x - 1 is complete
         const int xd = x - 1;
-        C h[Q], F[3], rho, u[3];
+        S h[Q];
+        C F[3], rho, u[3];
         static_for<Q>([&](auto ic) {
           constexpr int i = decltype(ic)::value;
-          h[i] = to_compute<L, i, S, C>(cel<L, i, 0>() < 0 ? g[i] : wait[k][i]);
+          h[i] = cel<L, i, 0>() < 0 ? g[i] : wait[k][i];
         });
         force_at(c, xd, F);
         const unsigned cell = (unsigned)((y0 + row_of(c) - 1) * a.nz + (z0 + z - rim_z)) *
                               (unsigned)sizeof(S);
-        bgk_collide_fast<L, C, FS, EQ, SH>(a, h, F, rho, u, [&](auto ic, C v) {
+        bgk_collide_stored<L, S, C, FS, EQ, SH>(a, h, F, rho, u, [&](auto ic, S v) {
           constexpr int i = decltype(ic)::value;
           char* base = reinterpret_cast<char*>(dst + (size_t)i * (size_t)a.N + (size_t)xd * plane);
-          store_pop<L, i, S, C>(reinterpret_cast<S*>(base + cell), v);
+          __builtin_nontemporal_store(v, reinterpret_cast<S*>(base + cell));
         });
       }
       static_for<Q>([&](auto ic) {

@@ -19,7 +19,7 @@
 //
 // Measured, microseconds a step, one-step kernel -> this one: 128^2 FP64 4.4 -> 2.0, FP32
 // 4.5 -> 1.4 (a step of a tile is 1.3 us of dependent FP64 instructions in one
-// wavefront a SIMD); 2048^2 FP32 55 -> 23, FP64 113 -> 82, FP16 38 -> 23: bound by the
+// wavefront a SIMD); 2048^2 FP32 55 -> 23, FP64 113 -> 82, FP16 38 -> 21: bound by the
 // vector instructions (five steps with a force field in FP32, 164 us: 80 % of the issue
 // slots, a quarter of the work in halos; with the parities chosen at run time 184 us).
 #pragma once
@@ -127,15 +127,10 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
           p[i] = lds[at[i]];
         });
       }
-      C f[Q], rho, u[3];
-      static_for<Q>([&](auto ic) {
-        constexpr int i = decltype(ic)::value;
-        f[i] = to_compute<L, i, S, C>(p[i]);
-      });
+      C rho, u[3];
       S v[Q];
-      bgk_collide_fast<L, C, FS, EQ, SH>(a, f, F, rho, u, [&](auto ic, C s) {
-        constexpr int i = decltype(ic)::value;
-        v[i] = to_storage<L, i, S, C>(s);
+      bgk_collide_stored<L, S, C, FS, EQ, SH>(a, p, F, rho, u, [&](auto ic, S s) {
+        v[decltype(ic)::value] = s;
       });
       if constexpr (last) {
         static_for<Q>([&](auto ic) {
