@@ -106,7 +106,7 @@ enum {
                              alpha = 2 (Collision.h:328-349).  Like the
                              reference's loop it bounds alpha only at
                              convergence, so it falls back exactly where the
-                             reference Newton does; one launch */
+                             reference Newton does */
 };
 
 typedef struct {
@@ -231,7 +231,11 @@ int lbm_get_alpha(lbm_handle *h, double *alpha);
 /* Advances nsteps fused collide-and-stream-pull steps (Routine.h:121-147,
  * Algorithm.h:326-358).  If store_last is nonzero the last step also writes
  * the output fields rho, u_hydro, alpha, force as storeFields does
- * (Algorithm.h:150-194).  Asynchronous on the handle's stream. */
+ * (Algorithm.h:150-194).  Asynchronous on the handle's stream.  With the
+ * automatic kernel choice one launch may take several of the steps; the
+ * populations end in the lattice that one launch a step would leave them in
+ * (lbm_device_populations).  In FP64 the result does not depend on how steps
+ * are split over calls; in FP32 and FP16 it does, by rounding. */
 int lbm_step(lbm_handle *h, int nsteps, int store_last);
 
 /* Copies the fields written by the last storing step: rho[N],
