@@ -806,10 +806,12 @@ __global__ void __launch_bounds__(BLOCK)
         }
       }
       // The sample log records the Newton solves: every solve of the Newton
-      // modes, of the correction modes those it deferred to MODE 3 (the cells
-      // the network or the stored alpha missed -- data to retrain on).
-      if constexpr (Shape::NIN > 0 && MODE != 1 && MODE != 2) {
-        if (a.log_cap > 0 && branch == 2 && (!groups || threadIdx.x % kGroupLanes == 0) &&
+      // modes, of the correction modes those that the correction left to Newton,
+      // here (3D) or in the list launch (the cells the network or the stored
+      // alpha missed -- data to retrain on).
+      if constexpr (Shape::NIN > 0 && (SERIES || (MODE != 1 && MODE != 2))) {
+        if (a.log_cap > 0 && branch == 2 && !first &&
+            (!groups || threadIdx.x % kGroupLanes == 0) &&
             sample_hash((unsigned)cell, a.log_salt) < a.log_threshold) {
           const unsigned long long k = atomicAdd(a.log_count, 1ull);
           if ((long long)k < a.log_cap) {
