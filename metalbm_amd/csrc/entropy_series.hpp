@@ -122,11 +122,14 @@ __device__ __forceinline__ CellRange cell_range(const V& p) {
 
 // The deviation test max |n| / f <= 1e-3 (Collision.h:284-303).  The FP32
 // ratio is good to 1e-6, so only a lane within 0.1% of the threshold, or one
-// with a population that is not clearly positive, is decided in FP64.
+// with a population that is not clearly positive, is decided in FP64; so is one
+// whose moments are not a number, which cell_range's maxima pass over (every n_i
+// is then not a number, n_0 among them).
 template <class L, class V>
 __device__ __forceinline__ bool small_deviation(const V& p, const CellRange& c) {
   bool small = !(c.x > 1.0e-3f);
-  if (!(c.f > 1.0e-30f) || fabsf(c.x - 1.0e-3f) <= 1.0e-6f) {
+  const float n0 = p.template n32<0>();
+  if (!(c.f > 1.0e-30f) || fabsf(c.x - 1.0e-3f) <= 1.0e-6f || n0 != n0) {
     small = true;
     static_for<L::dimQ>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
