@@ -105,6 +105,20 @@ __device__ __forceinline__ double log_or_nan(double v) {
 struct CellRange {
   float x = 0.0f, y = 0.0f, f = 3.0e38f;
 };
+// f is formed as (f - w) + w, with an error of up to 2^-23 (w + f): a cell's ratios are
+// good to 3e-4 where every f is above 5e-4 of the largest weight (a population of
+// the smallest weight then still reaches down to 3% of it).  Elsewhere, populations
+// at or below zero among them, the cell is decided in FP64.
+template <class L>
+constexpr float largest_weight() {
+  double w = 0.0;
+  for (int i = 0; i < L::dimQ; ++i) w = L::W[i] > w ? L::W[i] : w;
+  return float(w);
+}
+template <class L>
+__device__ __forceinline__ bool ratios_hold(const CellRange& c) {
+  return c.f > 5.0e-4f * largest_weight<L>();
+}
 template <class L, class V>
 __device__ __forceinline__ CellRange cell_range(const V& p) {
   CellRange c;
@@ -120,16 +134,15 @@ __device__ __forceinline__ CellRange cell_range(const V& p) {
   return c;
 }
 
-// The deviation test max |n| / f <= 1e-3 (Collision.h:284-303).  The FP32
-// ratio is good to 1e-6, so only a lane within 0.1% of the threshold, or one
-// with a population that is not clearly positive, is decided in FP64; so is one
+// The deviation test max |n| / f <= 1e-3 (Collision.h:284-303).  Where the FP32
+// ratios hold only a lane within 0.1% of the threshold is decided in FP64; so is one
 // whose moments are not a number, which cell_range's maxima pass over (every n_i
 // is then not a number, n_0 among them).
 template <class L, class V>
 __device__ __forceinline__ bool small_deviation(const V& p, const CellRange& c) {
   bool small = !(c.x > 1.0e-3f);
   const float n0 = p.template n32<0>();
-  if (!(c.f > 1.0e-30f) || fabsf(c.x - 1.0e-3f) <= 1.0e-6f || n0 != n0) {
+  if (!ratios_hold<L>(c) || fabsf(c.x - 1.0e-3f) <= 1.0e-6f || n0 != n0) {
     small = true;
     static_for<L::dimQ>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
@@ -371,7 +384,7 @@ __device__ __forceinline__ bool with_entropy_series(const V& p, const CellRange&
     s.build(p, c.y, stored);
     body(s);
   };
-  if (!(c.f > 1.0e-30f) || !(c.x < 0.39f)) return false;
+  if (!ratios_hold<L>(c) || !(c.x < 0.39f)) return false;
   if constexpr (L::dimQ <= 9) {
     using At = std::integral_constant<int, CENTRE_F>;
     const float r = 2.15f * c.x;

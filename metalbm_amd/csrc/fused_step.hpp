@@ -741,7 +741,7 @@ __global__ void __launch_bounds__(BLOCK)
                                                                   branch, its);
       } else if constexpr (MODE == 3 || (FLAT && MODE == 4)) {
         // alphaMax is its cap 2.5 where every |n| / f is below 0.4
-        if (!(range.x < 0.39f && range.f > 1.0e-30f) && alpha_capped<L, false>(p, alpha, amax))
+        if (!(range.x < 0.39f && ratios_hold<L>(range)) && alpha_capped<L, false>(p, alpha, amax))
           branch = 1;
         else
           alpha = newton_residual<L>(p, amax, stored, a.residual_tol, branch, its);
@@ -791,7 +791,7 @@ __global__ void __launch_bounds__(BLOCK)
         if constexpr (MODE == 2) start = stored;
         bool accepted = false;
         EvalCurv cv{};
-        if (!(range.x < 0.39f && range.f > 1.0e-30f) && alpha_capped<L, false>(p, alpha, amax)) {
+        if (!(range.x < 0.39f && ratios_hold<L>(range)) && alpha_capped<L, false>(p, alpha, amax)) {
           branch = 1;
         } else {
           accepted = residual_correction<L>(p, amax, start, a.residual_tol, alpha, its, cv);
