@@ -63,8 +63,9 @@ struct lbm_handle {
   uint64_t fields_version = 0;  // bumped whenever the fields are rewritten
   double* staging = nullptr;   // N doubles
   double* reduce_buf = nullptr;
-  char* ring = nullptr;     // pinned chunks of lbm_get_fields, and their events
+  char* ring = nullptr;     // pinned chunks of lbm_get_fields, their events and stream
   hipEvent_t ring_event[kRingSlots] = {};
+  hipStream_t ring_stream = nullptr;
   void* ftab[3] = {nullptr, nullptr, nullptr};
   int fax[3] = {3, 3, 3};
   unsigned long long* stats = nullptr;  // kStatSlots x kStatStride counters
@@ -311,6 +312,9 @@ int ensure_fields(lbm_handle* h) {
 // way while it copies the other (35 MB, ten steps of D3Q19 96 x 80 x 72 and the copy:
 // 3.41 -> 1.70 ms; 94 MB: 9.8 -> 4.1; 12 MB: 0.90 -> 0.63).  Requests of fewer bytes
 // than the pinned memory, and pinned or device destinations, are copied directly.
+// The calling thread waits for the handle's stream before the others start, and the
+// chunks go through a stream of their own: a handle's stream may be hipStreamPerThread,
+// which is another stream in each thread.
 struct FieldPart {
   char* dst;
   const char* src;
@@ -323,6 +327,8 @@ bool ensure_ring(lbm_handle* h) {
   for (int k = 0; ok && k < kRingSlots; ++k)
     if (!h->ring_event[k])
       ok = hipEventCreateWithFlags(&h->ring_event[k], hipEventDisableTiming) == hipSuccess;
+  if (ok && !h->ring_stream)
+    ok = hipStreamCreateWithFlags(&h->ring_stream, hipStreamNonBlocking) == hipSuccess;
   if (ok) {
     h->ring = mem;
   } else {
@@ -338,6 +344,7 @@ bool pageable(const void* p) {
   return true;
 }
 hipError_t copy_through_ring(lbm_handle* h, const FieldPart* parts, int n_parts) {
+  if (const hipError_t e = hipStreamSynchronize(h->stream); e != hipSuccess) return e;
   std::atomic<size_t> next{0};
   std::atomic<int> error{hipSuccess};
   auto chunk = [&](size_t k, FieldPart* c) {
@@ -358,8 +365,8 @@ hipError_t copy_through_ring(lbm_handle* h, const FieldPart* parts, int n_parts)
       if (error != hipSuccess || !chunk(next++, &c[k])) return false;
       const int slot = 2 * w + k;
       hipError_t e = hipMemcpyAsync(h->ring + slot * kRingChunk, c[k].src, c[k].bytes,
-                                    hipMemcpyDeviceToHost, h->stream);
-      if (e == hipSuccess) e = hipEventRecord(h->ring_event[slot], h->stream);
+                                    hipMemcpyDeviceToHost, h->ring_stream);
+      if (e == hipSuccess) e = hipEventRecord(h->ring_event[slot], h->ring_stream);
       if (e != hipSuccess) error = e;
       return e == hipSuccess;
     };
@@ -387,7 +394,8 @@ hipError_t copy_through_ring(lbm_handle* h, const FieldPart* parts, int n_parts)
   work(0);
   for (auto& t : helpers)
     if (t.joinable()) t.join();
-  const hipError_t e = hipStreamSynchronize(h->stream);
+  // every chunk has been waited for, unless one failed
+  const hipError_t e = hipStreamSynchronize(h->ring_stream);
   return error != hipSuccess ? (hipError_t)error.load() : e;
 }
 
@@ -419,6 +427,7 @@ void release(lbm_handle* h) {
   if (h->ring) (void)hipHostFree(h->ring);
   for (hipEvent_t e : h->ring_event)
     if (e) (void)hipEventDestroy(e);
+  if (h->ring_stream) (void)hipStreamDestroy(h->ring_stream);
   lbm::release_spectral(h->spectral);
   h->spectral = nullptr;
   if (h->ffield) {  // ftab points into the force field
