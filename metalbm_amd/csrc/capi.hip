@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -43,10 +44,6 @@ const Registry& registry() {
 }
 }  // namespace lbm
 
-// Pinned chunks, two to a copying thread.
-constexpr int kRingSlots = 8;
-constexpr size_t kRingChunk = 1 << 20;
-
 struct lbm_handle {
   lbm_config cfg{};
   int device = 0;           // the HIP device current at lbm_create
@@ -63,9 +60,6 @@ struct lbm_handle {
   uint64_t fields_version = 0;  // bumped whenever the fields are rewritten
   double* staging = nullptr;   // N doubles
   double* reduce_buf = nullptr;
-  char* ring = nullptr;     // pinned chunks of lbm_get_fields, their events and stream
-  hipEvent_t ring_event[kRingSlots] = {};
-  hipStream_t ring_stream = nullptr;
   void* ftab[3] = {nullptr, nullptr, nullptr};
   int fax[3] = {3, 3, 3};
   unsigned long long* stats = nullptr;  // kStatSlots x kStatStride counters
@@ -320,22 +314,78 @@ struct FieldPart {
   const char* src;
   size_t bytes;
 };
-bool ensure_ring(lbm_handle* h) {
-  if (h->ring) return true;
+// Pinned chunks, two to a copying thread, with their events and stream.  A process
+// has at most kRings of them, whichever handles use them (a call that finds all in
+// use copies directly), and frees them with its last handle.
+constexpr int kRingSlots = 8, kRings = 4;
+constexpr size_t kRingChunk = 1 << 20;
+struct FieldRing {
+  int device = -1;
   char* mem = nullptr;
-  bool ok = hipHostMalloc(&mem, kRingSlots * kRingChunk, hipHostMallocDefault) == hipSuccess;
-  for (int k = 0; ok && k < kRingSlots; ++k)
-    if (!h->ring_event[k])
-      ok = hipEventCreateWithFlags(&h->ring_event[k], hipEventDisableTiming) == hipSuccess;
-  if (ok && !h->ring_stream)
-    ok = hipStreamCreateWithFlags(&h->ring_stream, hipStreamNonBlocking) == hipSuccess;
-  if (ok) {
-    h->ring = mem;
-  } else {
-    (void)hipGetLastError();
-    if (mem) (void)hipHostFree(mem);
+  hipStream_t stream = nullptr;
+  hipEvent_t event[kRingSlots] = {};
+};
+struct RingPool {
+  std::mutex mu;
+  FieldRing* idle[kRings] = {};
+  int n_idle = 0, n_rings = 0, n_handles = 0;
+};
+RingPool g_rings;
+
+void free_ring(FieldRing* r) {
+  for (hipEvent_t e : r->event)
+    if (e) (void)hipEventDestroy(e);
+  if (r->stream) (void)hipStreamDestroy(r->stream);
+  if (r->mem) (void)hipHostFree(r->mem);
+  delete r;
+}
+// A ring of the current device, or NULL.
+FieldRing* take_ring(int device) {
+  RingPool& p = g_rings;
+  FieldRing* other = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(p.mu);
+    for (int k = 0; k < p.n_idle; ++k)
+      if (p.idle[k]->device == device) {
+        FieldRing* r = p.idle[k];
+        p.idle[k] = p.idle[--p.n_idle];
+        return r;
+      }
+    if (p.n_rings < kRings)
+      ++p.n_rings;
+    else if (p.n_idle > 0)
+      other = p.idle[--p.n_idle];  // another device's: its place is taken
+    else
+      return nullptr;
   }
-  return ok;
+  if (other) free_ring(other);
+  FieldRing* r = new (std::nothrow) FieldRing;
+  bool ok = r && hipHostMalloc(&r->mem, kRingSlots * kRingChunk, hipHostMallocDefault) == hipSuccess;
+  ok = ok && hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking) == hipSuccess;
+  for (int k = 0; ok && k < kRingSlots; ++k)
+    ok = hipEventCreateWithFlags(&r->event[k], hipEventDisableTiming) == hipSuccess;
+  if (ok) {
+    r->device = device;
+    return r;
+  }
+  (void)hipGetLastError();
+  if (r) free_ring(r);
+  std::lock_guard<std::mutex> lock(p.mu);
+  --p.n_rings;
+  return nullptr;
+}
+void give_ring(FieldRing* r) {
+  std::lock_guard<std::mutex> lock(g_rings.mu);
+  g_rings.idle[g_rings.n_idle++] = r;
+}
+// Counts a process's handles; the last one takes the rings with it.
+void count_handle(int change) {
+  std::lock_guard<std::mutex> lock(g_rings.mu);
+  g_rings.n_handles += change;
+  while (g_rings.n_handles == 0 && g_rings.n_idle > 0) {
+    free_ring(g_rings.idle[--g_rings.n_idle]);
+    --g_rings.n_rings;
+  }
 }
 bool pageable(const void* p) {
   hipPointerAttribute_t at{};
@@ -343,7 +393,8 @@ bool pageable(const void* p) {
   (void)hipGetLastError();  // memory that HIP does not know
   return true;
 }
-hipError_t copy_through_ring(lbm_handle* h, const FieldPart* parts, int n_parts) {
+hipError_t copy_through_ring(lbm_handle* h, FieldRing& ring, const FieldPart* parts,
+                             int n_parts) {
   if (const hipError_t e = hipStreamSynchronize(h->stream); e != hipSuccess) return e;
   std::atomic<size_t> next{0};
   std::atomic<int> error{hipSuccess};
@@ -364,9 +415,9 @@ hipError_t copy_through_ring(lbm_handle* h, const FieldPart* parts, int n_parts)
     auto issue = [&](int k) {
       if (error != hipSuccess || !chunk(next++, &c[k])) return false;
       const int slot = 2 * w + k;
-      hipError_t e = hipMemcpyAsync(h->ring + slot * kRingChunk, c[k].src, c[k].bytes,
-                                    hipMemcpyDeviceToHost, h->ring_stream);
-      if (e == hipSuccess) e = hipEventRecord(h->ring_event[slot], h->ring_stream);
+      hipError_t e = hipMemcpyAsync(ring.mem + slot * kRingChunk, c[k].src, c[k].bytes,
+                                    hipMemcpyDeviceToHost, ring.stream);
+      if (e == hipSuccess) e = hipEventRecord(ring.event[slot], ring.stream);
       if (e != hipSuccess) error = e;
       return e == hipSuccess;
     };
@@ -375,12 +426,12 @@ hipError_t copy_through_ring(lbm_handle* h, const FieldPart* parts, int n_parts)
     for (int k = 0; have; k ^= 1) {
       have = issue(k ^ 1);
       const int slot = 2 * w + k;
-      const hipError_t e = hipEventSynchronize(h->ring_event[slot]);
+      const hipError_t e = hipEventSynchronize(ring.event[slot]);
       if (e != hipSuccess) {
         error = e;
         break;
       }
-      std::memcpy(c[k].dst, h->ring + slot * kRingChunk, c[k].bytes);
+      std::memcpy(c[k].dst, ring.mem + slot * kRingChunk, c[k].bytes);
     }
   };
   std::thread helpers[kRingSlots / 2];
@@ -395,7 +446,7 @@ hipError_t copy_through_ring(lbm_handle* h, const FieldPart* parts, int n_parts)
   for (auto& t : helpers)
     if (t.joinable()) t.join();
   // every chunk has been waited for, unless one failed
-  const hipError_t e = hipStreamSynchronize(h->ring_stream);
+  const hipError_t e = hipStreamSynchronize(ring.stream);
   return error != hipSuccess ? (hipError_t)error.load() : e;
 }
 
@@ -424,10 +475,6 @@ hipError_t seed_state(lbm_handle* h, const double* drho, double rho0, const doub
 }
 
 void release(lbm_handle* h) {
-  if (h->ring) (void)hipHostFree(h->ring);
-  for (hipEvent_t e : h->ring_event)
-    if (e) (void)hipEventDestroy(e);
-  if (h->ring_stream) (void)hipStreamDestroy(h->ring_stream);
   lbm::release_spectral(h->spectral);
   h->spectral = nullptr;
   if (h->ffield) {  // ftab points into the force field
@@ -744,6 +791,7 @@ int lbm_create(const lbm_config* cfg, lbm_handle** out) {
       (void)hipGetLastError();  // no room for the list: see lists_cells
   }
   *out = h;
+  count_handle(1);
   return LBM_OK;
 }
 
@@ -752,6 +800,7 @@ int lbm_destroy(lbm_handle* h) {
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   release(h);
   delete h;
+  count_handle(-1);
   return LBM_OK;
 }
 
@@ -1162,8 +1211,9 @@ int lbm_get_fields(lbm_handle* h, double* rho, double* u_hydro, double* alpha,
     int current = -1;
     HIP_TRY(h, hipGetDevice(&current));
     if (current != h->device) HIP_TRY(h, hipSetDevice(h->device));
-    const bool ring = ensure_ring(h);
-    const hipError_t e = ring ? copy_through_ring(h, parts, n_parts) : hipSuccess;
+    FieldRing* ring = take_ring(h->device);
+    const hipError_t e = ring ? copy_through_ring(h, *ring, parts, n_parts) : hipSuccess;
+    if (ring) give_ring(ring);
     if (current != h->device) (void)hipSetDevice(current);
     HIP_TRY(h, e);
     if (ring) return LBM_OK;
