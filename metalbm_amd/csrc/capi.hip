@@ -505,12 +505,12 @@ bool certified_mode(const lbm_handle* h) {
 
 // Whether a step lists cells for a second launch (see k_elbm): the certified
 // modes always; on larger domains the Newton modes in 3D and the reference
-// Newton in D2Q9, where the list exists (it is allocated with the handle;
-// without the memory for it the term-by-term kernels solve every cell).  The
-// parity build's reference Newton never does.
+// Newton in D2Q9, where the list exists (it is allocated with the handle or when
+// such a mode is set; without the memory for it the term-by-term kernels solve
+// every cell).  The parity build's reference Newton never does.
 bool newton_lists(const lbm_handle* h) {
   const bool parity = h->ctype == TYPE_F64 && !h->cfg.shifted;
-  if (h->alpha_mode == LBM_ALPHA_NEWTON && parity) return false;
+  if (certified_mode(h) || (h->alpha_mode == LBM_ALPHA_NEWTON && parity)) return false;
   return h->D == 3 ? h->N >= kListMinCells3D
                    : h->alpha_mode == LBM_ALPHA_NEWTON && h->N >= kListMinCells2D;
 }
@@ -538,6 +538,11 @@ hipError_t allocate_list(lbm_handle* h) {
     e = hipMalloc(&h->defer_list,
                   (size_t)list_shards(h) * (size_t)list_capacity(h) * sizeof(int));
   return e;
+}
+
+// For a Newton mode that lists cells, if there is room (see lists_cells).
+void allocate_newton_list(lbm_handle* h) {
+  if (newton_lists(h) && allocate_list(h) != hipSuccess) (void)hipGetLastError();
 }
 
 StepArgs make_args(const lbm_handle* h) {
@@ -786,9 +791,7 @@ int lbm_create(const lbm_config* cfg, lbm_handle** out) {
       h->err = std::string("alpha field: ") + hipGetErrorString(e);
       return bail(LBM_E_HIP);
     }
-    if (h->N >= (h->D == 3 ? kListMinCells3D : kListMinCells2D) &&
-        allocate_list(h) != hipSuccess)
-      (void)hipGetLastError();  // no room for the list: see lists_cells
+    allocate_newton_list(h);
   }
   *out = h;
   count_handle(1);
@@ -1791,6 +1794,7 @@ int lbm_set_alpha_mode(lbm_handle* h, int mode, double residual_tol) {
     return fail(h, LBM_E_INVALID, "residual_tol must be positive");
   h->alpha_mode = mode;
   if (residual_tol > 0.0) h->residual_tol = residual_tol;
+  allocate_newton_list(h);
   return LBM_OK;
 }
 
