@@ -38,6 +38,7 @@
 // the term-by-term solver.
 #pragma once
 
+#include "entropy_log.hpp"
 #include "mlp.hpp"
 
 namespace lbm {
@@ -52,52 +53,6 @@ constexpr double kSeriesReach = CENTRE == CENTRE_F   ? (K == 10 ? 0.0262 : 0.258
 
 // Populations of the 3D pass in flight together.
 constexpr int kSeriesGroup = 9;
-
-// n / v to about an ulp for v > 0 in the normal range: the hardware reciprocal
-// with one Newton-Raphson correction (to 2^-48 or better) and the quotient's
-// residual through it.
-__device__ __forceinline__ double quotient(double n, double v) {
-  double r = __builtin_amdgcn_rcp(v);
-  r = fma(r, fma(-v, r, 1.0), r);
-  const double q = n * r;
-  return fma(r, fma(-v, q, n), q);
-}
-
-// log(1 + y) for 1 + y positive and normal: 1 + y = 2^k m with m in
-// [sqrt(1/2), sqrt(2)), log m = 2 atanh(s), s = (m - 1) / (m + 1), s^2 <=
-// 0.02944; at k = 0, m - 1 is y itself, so nothing is lost for small y.  The
-// atanh series beyond its first term is replaced by the polynomial through
-// seven Chebyshev nodes of that interval (relative error of the logarithm
-// below 5e-18), so the result is within about an ulp, as the library's is, at
-// a third of its instructions.
-__device__ __forceinline__ double log1p_positive(double y) {
-  const double v = 1.0 + y;
-  double m = __builtin_amdgcn_frexp_mant(v);  // [1/2, 1)
-  int k = __builtin_amdgcn_frexp_exp(v);
-  const bool low = m < 0.70710678118654752440;
-  m = low ? m + m : m;
-  k = low ? k - 1 : k;
-  const double m1 = k == 0 ? y : m - 1.0;
-  const double s = quotient(m1, m1 + 2.0);
-  const double z = s * s;
-  double p = 0.146167211662876;
-  p = fma(p, z, 0.15331699634642276);
-  p = fma(p, z, 0.1818288978615799);
-  p = fma(p, z, 0.22222211125723262);
-  p = fma(p, z, 0.28571428626031065);
-  p = fma(p, z, 0.3999999999989938);
-  p = fma(p, z, 0.666666666666667);
-  // ln 2 in two parts, the first short enough for k ln2_hi to be exact
-  constexpr double ln2_hi = 0x1.62e42fee00000p-1, ln2_lo = 0x1.a39ef35793c76p-33;
-  const double dk = double(k);
-  return fma(dk, ln2_hi, fma(dk, ln2_lo, fma(s * z, p, s + s)));
-}
-// log(v) for any v: not a number for v <= 0 (the library's -inf at 0 enters G
-// as 0 times infinity).
-__device__ __forceinline__ double log_or_nan(double v) {
-  const double l = log1p_positive(v - 1.0);
-  return v > 0.0 ? l : __builtin_nan("");
-}
 
 // First look at one cell in FP32: the largest |n| / f, the smallest f and (D2Q9)
 // the largest |f / w - 1|.  It settles the deviation test away from its threshold
