@@ -234,8 +234,8 @@ int lbm_get_alpha(lbm_handle *h, double *alpha);
  * (Algorithm.h:150-194).  Asynchronous on the handle's stream.  With the
  * automatic kernel choice one launch may take several of the steps; the
  * populations end in the lattice that one launch a step would leave them in
- * (lbm_device_populations).  In FP64 the result does not depend on how steps
- * are split over calls; in FP32 and FP16 it does, by rounding. */
+ * (lbm_device_populations).  The result does not depend on how steps are split
+ * over calls. */
 int lbm_step(lbm_handle *h, int nsteps, int store_last);
 
 /* Copies the fields written by the last storing step: rho[N],

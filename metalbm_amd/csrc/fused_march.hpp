@@ -12,8 +12,8 @@
 // two steps read the lattice once (plus the rims) and write it once.
 //
 // The intermediate populations are rounded to the storage type and every cell
-// collides with the one-step kernels' operators, so the result is that of two
-// one-step launches up to the rounding of FP32 sums.
+// collides as in the one-step kernels, so the result is that of two one-step
+// launches to the bit.
 //
 // Tile: with the three populations that stay in their column held in
 // registers, a column takes Q - 3 values of LDS, and the CU's 160 KB hold 2560
@@ -37,7 +37,8 @@
 // populations packed in pairs: 1162 against 1205, 72 % of the issue slots at half the
 // bytes, but 192^3 1.01 to 1.21 and 64^3 2.2 times the one-step kernel's time) stays
 // with the one-step kernels, and so does FP64 storage with FP32 arithmetic, whose
-// populations would show that the two kernels round their FP32 sums differently.
+// kernels collide one population at a time: the pairwise form rounds its sums in
+// another order, which FP64 populations show (1.7e-6 of them).
 #pragma once
 
 #include "fused_step.hpp"

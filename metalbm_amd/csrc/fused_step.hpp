@@ -28,8 +28,12 @@ __device__ __forceinline__ void store_fields(const StepArgs& a, int cell, int FS
   } else {
     // Generic: u + 0.5 / rho * F (ForcingScheme.h:26-33)
     const C h = C(0.5) / rho;
-    for (int d = 0; d < L::dimD; ++d)
-      a.uh_out[(size_t)d * a.N + cell] = double(u[d] + F[d] * h);
+    for (int d = 0; d < L::dimD; ++d) {
+      C v;
+      if constexpr (std::is_same_v<C, float>) v = fmaf(F[d], h, u[d]);  // the same in each kernel
+      else v = u[d] + F[d] * h;
+      a.uh_out[(size_t)d * a.N + cell] = double(v);
+    }
   }
   if (a.alpha_out) a.alpha_out[cell] = alpha;
   if (a.F_out)
@@ -47,12 +51,33 @@ constexpr int opposite() {
   return -1;
 }
 
-// Coefficients of scale (base + rho (P(cu) - 1)), P the Ma3 polynomial, split into
-// its even part e0 + cu^2 (e1 + e2 cu^2) and its odd part cu (o0 + o1 cu^2).
+// The single-precision BGK collision of one cell (Collision.h:134-151), two opposite
+// populations at a time: they share every term of the Ma3 equilibrium and of the
+// source up to the sign of the odd part (the two-step kernel on D3Q19 256^3 with the
+// Guo source: 179 million vector instructions a launch instead of 248, addresses
+// included).  Every kernel that one handle's steps may go through takes its arithmetic
+// from here, so that a result does not depend on how steps are split over launches and
+// calls.  For that each kernel has to round the same way, and the compiler, which in
+// these files fuses any product that feeds a sum (pragmas or not), must have no choice:
+// every fused operation is written out, and no rounded product is added or subtracted
+// except as the addend of one.  SC: populations are in their FP16 storage scales
+// (powers of two, so that the products with them, folded into the sums' and the results'
+// factors, round nothing).
+//
+// f + omega_eq (feq - f) rather than omega_f f + omega_eq feq: omega_f and omega_eq
+// rounded to single precision do not add up to 1, and that error, the same in every cell
+// and step, was most of the result's.  (EDM: omega_f (f - feq) + feq(v), for the same
+// reason.)  Error against 64 bits after 15 steps of noise on D3Q19 with tau 0.55 / 0.6624
+// / 0.8 (relative 2-norm of f - w): 5.5e-7 / 2.5e-7 / 2.0e-7; with the two rates 9.5e-7 /
+// 8.4e-7 / 2.4e-7; one population at a time, as it was before the pairs, 9.6e-7 / 6.5e-7
+// / 2.8e-7; D2Q9, 2000 steps, tau 0.53: 1.7e-5, 8.9e-5 and 9.1e-5.
+
+// Ma3: t(cu) = base + rho (P(cu) - 1), P the polynomial (Equilibrium.h:17-33), times
+// `scale`, split into its even part e0 + cu^2 (e1 + e2 cu^2) and its odd part
+// cu (o0 + o1 cu^2).
 struct Ma3Split {
   float e0, e1, e2, o0, o1;
-  __device__ __forceinline__ Ma3Split(float scale, float rho, float base, float u2) {
-#pragma clang fp contract(off)
+  __device__ __forceinline__ void set(float scale, float rho, float base, float u2) {
     const float sr = scale * rho;
     e0 = fmaf(sr, u2 * fmaf(1.125f, u2, -1.5f), scale * base);
     e1 = sr * fmaf(-6.75f, u2, 4.5f);
@@ -63,89 +88,172 @@ struct Ma3Split {
   __device__ __forceinline__ float even(float q, float more) const {
     return fmaf(q, fmaf(q, e2, e1), more);
   }
-  __device__ __forceinline__ float odd(float cu, float q, float more) const {
-    return fmaf(cu, fmaf(q, o1, o0), more);
+  __device__ __forceinline__ float odd(float q) const { return fmaf(q, o1, o0); }
+};
+
+// Product equilibrium: ExactShifted's factors e[d][c + 1] = phi_d^c - 1 with its fused
+// operations written out.
+template <class L>
+struct ExactTerms {
+  float e[3][3];
+  __device__ __forceinline__ void set(const float* u) {
+    for (int d = 0; d < L::dimD; ++d) {
+      const float v = u[d], t = 3.0f * v;
+      const float s = sqrtf(fmaf(t, v, 1.0f)), sm1 = (t * v) / (1.0f + s);
+      e[d][1] = -sm1;
+      e[d][2] = fmaf(v, fmaf(-2.0f, s, 5.0f), fmaf(2.0f, sm1, -(t * v))) / (1.0f - v);
+      e[d][0] = fmaf(v, s, fmaf(-4.0f, v, -2.0f * sm1)) / fmaf(2.0f, v, s);
+    }
+  }
+  template <int i>
+  __device__ __forceinline__ float p() const {
+    const float e0 = e[0][cel<L, i, 0>() + 1], e1 = e[1][cel<L, i, 1>() + 1];
+    float t = fmaf(e0, e1, e0 + e1);
+    if constexpr (L::dimD == 3) {
+      const float e2 = e[2][cel<L, i, 2>() + 1];
+      t = fmaf(t, e2, t + e2);
+    }
+    return t;
   }
 };
 
-// The single-precision Ma3 collision, two opposite populations at a time: they
-// share every term of the equilibrium and of the source up to the sign of the
-// odd part, and the relaxation rate and the source are folded into the
-// polynomial's coefficients once per cell (the two-step kernel on D3Q19 256^3 with
-// the Guo source: 179 million vector instructions a launch instead of 248, addresses
-// included).  Contraction is off and every fused operation is written out, so each
-// kernel that inlines this gets the same bits.  SC: f and the results are in the
-// populations' FP16 storage scales (powers of two, so that the products with them,
-// folded into the sums' and the results' factors, round nothing).
-template <class L, int FS, bool SH, bool SC, class EMIT>
-__device__ __forceinline__ void bgk_collide_pairs(const StepArgs& a, const float* f,
-                                                  const float* F, float& rho, float* u,
-                                                  EMIT&& emit) {
-#pragma clang fp contract(off)
-  constexpr int Q = L::dimQ, D = L::dimD;
-  const float of = float(a.omega_f), oe = float(a.omega_eq), g3 = float(3.0 * a.guo_coef);
-  constexpr float s0 = SC ? float(kHalfScale<L, 0>) : 1.0f;
-  float sum = f[0] * (1.0f / s0), j[3] = {0.0f, 0.0f, 0.0f};
-  static_for<Q>([&](auto ic) {
-    constexpr int i = decltype(ic)::value, o = opposite<L, i>();
-    if constexpr (i < o) {
-      constexpr float inv = SC ? float(1.0 / kHalfScale<L, i>) : 1.0f;
-      sum = SC ? fmaf(f[i] + f[o], inv, sum) : sum + (f[i] + f[o]);
-      const float d = SC ? (f[i] - f[o]) * inv : f[i] - f[o];
-      static_for<D>([&](auto dc) {
-        constexpr int c = L::C[i][decltype(dc)::value];
-        if constexpr (c > 0) j[decltype(dc)::value] += d;
-        if constexpr (c < 0) j[decltype(dc)::value] -= d;
-      });
-    }
-  });
-  rho = SH ? 1.0f + sum : sum;
-  const float r0 = __builtin_amdgcn_rcpf(rho);
-  const float rr = fmaf(r0, fmaf(-rho, r0, 1.0f), r0);  // see moments_shifted_scaled
-  u[2] = 0.0f;
-  for (int d = 0; d < D; ++d) u[d] = j[d] * rr;
-  auto square = [&](const float* v) {
-    float s = v[0] * v[0];
-    for (int d = 1; d < D; ++d) s = fmaf(v[d], v[d], s);
-    return s;
-  };
-  // EDM: omega_eq feq(u) + (feq(u + F / rho) - feq(u)) (ForcingScheme.h:184-197)
-  const float scale = FS == SRC_EDM ? float(a.omega_eq - 1.0) : oe;
-  Ma3Split E(scale, rho, sum, square(u));
-  float v[3] = {0.0f, 0.0f, 0.0f};
-  if constexpr (FS == SRC_EDM)
-    for (int d = 0; d < D; ++d) v[d] = fmaf(F[d], rr, u[d]);
-  const Ma3Split E2(1.0f, rho, sum, square(v));
-  // Guo: w 3 g (c.F - u.F + 3 (c.u) (c.F)), g = 1 - 1 / (2 tau) (ForcingScheme.h:99-117)
-  float G[3] = {0.0f, 0.0f, 0.0f};
-  if constexpr (FS == SRC_GUO) {
-    for (int d = 0; d < D; ++d) G[d] = g3 * F[d];
-    for (int d = 0; d < D; ++d) E.e0 = fmaf(-u[d], G[d], E.e0);
+template <class L, int FS, int EQ, bool SH, bool SC>
+struct PairCollision {
+  static constexpr bool MA3 = EQ == (int)EquilibriumType::TruncationMa3;
+  float rho, u[3];   // the moments
+  float of, oe, sum; // sum: drho (SH) or rho
+  float v[3];        // EDM: u + F / rho
+  float G[3], g, uG; // Guo: omega_eq w g (c.G - u.G + 3 (c.u) (c.G)), G = F, g =
+                     // 3 (1 - 1 / (2 tau)) / omega_eq (ForcingScheme.h:99-117), uG = g u.G
+  Ma3Split E, E2;
+  ExactTerms<L> X, X2;
+
+  template <int i>
+  static constexpr float scale_of() {
+    return SC ? float(kHalfScale<L, i>) : 1.0f;
   }
-  if constexpr (FS == SRC_EDM) E.e0 += E2.e0;
-  emit(std::integral_constant<int, 0>{}, fmaf(float(L::W[0]) * s0, E.e0, of * f[0]));
-  static_for<Q>([&](auto ic) {
-    constexpr int i = decltype(ic)::value, o = opposite<L, i>();
-    if constexpr (i < o) {
-      constexpr float w = float(L::W[i]) * (SC ? float(kHalfScale<L, i>) : 1.0f);
-      const float cu = cdot<L, i>(u), q = cu * cu;
-      float even = E.even(q, E.e0), odd;
-      if constexpr (FS == SRC_GUO) {
-        const float cG = cdot<L, i>(G);
-        even = fmaf(3.0f * cu, cG, even);
-        odd = E.odd(cu, q, cG);
-      } else if constexpr (FS == SRC_EDM) {
-        const float cv = cdot<L, i>(v), r = cv * cv;
-        even = E2.even(r, even);
-        odd = E.odd(cu, q, cv * fmaf(r, E2.o1, E2.o0));
-      } else {
-        odd = cu * fmaf(q, E.o1, E.o0);
+
+  __device__ __forceinline__ void set(const StepArgs& a, const float* f, const float* F) {
+    constexpr int Q = L::dimQ, D = L::dimD;
+    of = float(a.omega_f);
+    oe = float(a.omega_eq);
+    sum = f[0] * (1.0f / scale_of<0>());
+    float j[3] = {0.0f, 0.0f, 0.0f};
+    static_for<Q>([&](auto ic) {
+      constexpr int i = decltype(ic)::value, o = opposite<L, i>();
+      if constexpr (i < o) {
+        constexpr float inv = 1.0f / scale_of<i>();
+        sum = SC ? fmaf(f[i] + f[o], inv, sum) : sum + (f[i] + f[o]);
+        const float d = SC ? (f[i] - f[o]) * inv : f[i] - f[o];
+        static_for<D>([&](auto dc) {
+          constexpr int c = L::C[i][decltype(dc)::value];
+          if constexpr (c > 0) j[decltype(dc)::value] += d;
+          if constexpr (c < 0) j[decltype(dc)::value] -= d;
+        });
       }
-      emit(std::integral_constant<int, i>{}, fmaf(w, even + odd, of * f[i]));
-      emit(std::integral_constant<int, o>{}, fmaf(w, even - odd, of * f[o]));
+    });
+    rho = SH ? 1.0f + sum : sum;
+    // The reciprocal estimate with one correction, and each quotient's remainder
+    // through it: a biased 1 / rho biases every equilibrium velocity (see
+    // moments_shifted_scaled).
+    const float r0 = __builtin_amdgcn_rcpf(rho);
+    const float rr = fmaf(r0, fmaf(-rho, r0, 1.0f), r0);
+    u[2] = v[2] = 0.0f;
+    for (int d = 0; d < D; ++d) {
+      const float q = j[d] * rr;
+      u[d] = fmaf(rr, fmaf(-rho, q, j[d]), q);
     }
-  });
-}
+    if constexpr (FS == SRC_EDM)  // feq(rho, u + F / rho) - feq (ForcingScheme.h:184-197)
+      for (int d = 0; d < D; ++d) v[d] = fmaf(F[d], rr, u[d]);
+    uG = 0.0f;
+    if constexpr (FS == SRC_GUO) {
+      g = float(3.0 * a.guo_coef / a.omega_eq);
+      // summed by itself: taken from E.e0 term by term, its roundings moved the mean
+      // density by 1e-12 a step, always one way
+      for (int d = 0; d < D; ++d) {
+        G[d] = F[d];
+        uG = fmaf(u[d], g * F[d], uG);
+      }
+    }
+    if constexpr (MA3) {
+      auto square = [](const float* w) {
+        float s = w[0] * w[0];
+        for (int d = 1; d < D; ++d) s = fmaf(w[d], w[d], s);
+        return s;
+      };
+      E.set(FS == SRC_EDM ? -of : 1.0f, rho, sum, square(u));
+      if constexpr (FS == SRC_GUO) E.e0 -= uG;
+      if constexpr (FS == SRC_EDM) {
+        E2.set(1.0f, rho, sum, square(v));
+        E.e0 += E2.e0;
+      }
+    } else {
+      X.set(u);
+      if constexpr (FS == SRC_EDM) X2.set(v);
+    }
+  }
+
+  // Post-collision from the pulled f and t: feq / w - (SH ? 1 : 0) with the source (EDM:
+  // feq(v) / w ... - omega_f feq / w ...).
+  __device__ __forceinline__ float relaxed(float w, float t, float f) const {
+    if constexpr (FS == SRC_EDM) return fmaf(w, t, of * f);
+    else return fmaf(oe, fmaf(w, t, -f), f);
+  }
+  // t of the product equilibrium, without Guo's source.
+  template <int i>
+  __device__ __forceinline__ float exact() const {
+    const float t = fmaf(rho, X.template p<i>(), sum);
+    if constexpr (FS == SRC_EDM) return fmaf(-of, t, fmaf(rho, X2.template p<i>(), sum));
+    else return t;
+  }
+
+  // Population 0 and the pair i, opposite<L, i>().
+  __device__ __forceinline__ float rest(float f) const {
+    constexpr float w = float(L::W[0]) * scale_of<0>();
+    if constexpr (MA3) return relaxed(w, E.e0, f);
+    else return relaxed(w, FS == SRC_GUO ? exact<0>() - uG : exact<0>(), f);
+  }
+  template <int i>
+  __device__ __forceinline__ void pair(float fi, float fo, float& to_i, float& to_o) const {
+    constexpr int o = opposite<L, i>();
+    constexpr float w = float(L::W[i]) * scale_of<i>();
+    const float cu = cdot<L, i>(u);
+    float cG = 0.0f;
+    if constexpr (FS == SRC_GUO) cG = cdot<L, i>(G);  // of loaded values: no products
+    float ti, to;
+    if constexpr (MA3) {
+      const float q = cu * cu;
+      float even = E.even(q, E.e0);
+      if constexpr (FS == SRC_ZERO) {
+        const float odd = E.odd(q);
+        ti = fmaf(cu, odd, even);
+        to = fmaf(-cu, odd, even);
+      } else {
+        float odd;
+        if constexpr (FS == SRC_GUO) {
+          even = fmaf(3.0f * cu, g * cG, even);
+          odd = fmaf(cu, E.odd(q), g * cG);
+        } else {
+          const float cv = cdot<L, i>(v), r = cv * cv;
+          even = E2.even(r, even);
+          odd = fmaf(cu, E.odd(q), cv * E2.odd(r));
+        }
+        ti = even + odd;
+        to = even - odd;
+      }
+    } else {
+      ti = exact<i>();
+      to = exact<o>();
+      if constexpr (FS == SRC_GUO) {
+        const float even = fmaf(3.0f * cu, g * cG, -uG);
+        ti += fmaf(g, cG, even);
+        to += fmaf(-g, cG, even);
+      }
+    }
+    to_i = relaxed(w, ti, fi);
+    to_o = relaxed(w, to, fo);
+  }
+};
 
 // BGK collision of one cell (Collision.h:134-151): f the pulled populations, F the
 // force.  emit(i, v) takes the post-collision populations in order, v in the
@@ -227,15 +335,23 @@ __device__ __forceinline__ void bgk_collide(const StepArgs& a, const C* f, const
   }
 }
 
-// The form that the kernels of several steps take: stored populations to stored ones.
-// FP16 populations stay in their storage scales (D2Q9 2000^2, Guo: 23.8 -> 21.3 us a
-// step, 128^2 3% less, for two products a population less).
-template <class L, class S, class C, int FS, int EQ, bool SH, class EMIT>
+// Whether a number format has kernels of several steps (instantiate.hpp registers them
+// by this), and whether its collisions therefore take the pairwise form in every kernel.
+template <class L, class S, class C>
+constexpr bool kSeveralSteps = L::dimD == 3 ? std::is_same_v<S, C> : sizeof(S) <= sizeof(C);
+template <class L, class S, class C>
+constexpr bool kPairs = std::is_same_v<C, float> && kSeveralSteps<L, S, C>;
+
+// Stored populations to stored ones; emit(i, s) takes them, s in the storage type.  FP16
+// populations of the pairwise form stay in their storage scales (D2Q9 2000^2, Guo: 23.8
+// -> 21.3 us a step, 128^2 3% less, for two products a population less).  ORDERED: in the
+// order of the populations, for kernels that wait for memory (D3Q27 193 x 161 x 130, one
+// step, Guo with the product equilibrium: 269 us, 287 with each pair stored at once and
+// 298 with all at the end; the compiler shares a pair's terms or forms them twice).
+template <class L, class S, class C, int FS, int EQ, bool SH, bool ORDERED = false, class EMIT>
 __device__ __forceinline__ void bgk_collide_stored(const StepArgs& a, const S* p, const C* F,
                                                    C& rho, C* u, EMIT&& emit) {
-  constexpr bool PAIRS =
-      std::is_same_v<C, float> && EQ == (int)EquilibriumType::TruncationMa3;
-  constexpr bool SC = PAIRS && std::is_same_v<S, _Float16>;
+  constexpr bool SC = kPairs<L, S, C> && std::is_same_v<S, _Float16>;
   C f[L::dimQ];
   static_for<L::dimQ>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
@@ -245,10 +361,28 @@ __device__ __forceinline__ void bgk_collide_stored(const StepArgs& a, const S* p
     constexpr int i = decltype(ic)::value;
     emit(ic, SC ? S(v) : to_storage<L, i, S, C>(v));
   };
-  if constexpr (PAIRS)
-    bgk_collide_pairs<L, FS, SH, SC>(a, f, F, rho, u, stored);
-  else
+  if constexpr (kPairs<L, S, C>) {
+    PairCollision<L, FS, EQ, SH, SC> cell;
+    cell.set(a, f, F);
+    rho = cell.rho;
+    for (int d = 0; d < 3; ++d) u[d] = cell.u[d];
+    stored(std::integral_constant<int, 0>{}, cell.rest(f[0]));
+    static_for<L::dimQ>([&](auto ic) {
+      constexpr int i = decltype(ic)::value, o = opposite<L, i>();
+      float vi, vo;
+      if constexpr (ORDERED && i != o) {
+        if constexpr (i < o) cell.template pair<i>(f[i], f[o], vi, vo);
+        else cell.template pair<o>(f[o], f[i], vo, vi);
+        stored(ic, vi);
+      } else if constexpr (i < o) {
+        cell.template pair<i>(f[i], f[o], vi, vo);
+        stored(ic, vi);
+        stored(std::integral_constant<int, o>{}, vo);
+      }
+    });
+  } else {
     bgk_collide<L, C, FS, EQ, SH>(a, f, F, rho, u, stored);
+  }
 }
 
 template <class L, class S, class C, int FS, int EQ, bool SH, int BLOCK, bool NT>
@@ -259,14 +393,14 @@ __global__ void __launch_bounds__(BLOCK) k_bgk(const StepArgs a, int FSX) {
   const int cell = self_index<L>(a, c);
   S* __restrict__ dst = static_cast<S*>(a.dst);
 
-  C f[Q];
-  pull<L, S, C, NT>(a, c, f);
+  S f[Q];
+  pull_stored<L, S, NT>(a, c, f);
   C F[3];
   force_of_cell<L, C>(a, c, F);
   C rho, u[3];
-  bgk_collide<L, C, FS, EQ, SH>(a, f, F, rho, u, [&](auto ic, C v) {
+  bgk_collide_stored<L, S, C, FS, EQ, SH, true>(a, f, F, rho, u, [&](auto ic, S v) {
     constexpr int i = decltype(ic)::value;
-    store_pop<L, i, S, C>(dst + (size_t)i * a.N + cell, v);
+    __builtin_nontemporal_store(v, dst + (size_t)i * a.N + cell);
   });
   if (a.store) store_fields<L, C>(a, cell, FSX, rho, u, F, 2.0);
 }

@@ -12,7 +12,8 @@
 // active lane takes the value across the segment boundary from one extra
 // uniform load.
 //
-// Same arithmetic as k_bgk per cell (reference order for FP64 unshifted).
+// Same arithmetic as k_bgk per cell (reference order for FP64 unshifted, the pairwise
+// form to the bit for FP32).
 #pragma once
 
 #include "fused_step.hpp"
@@ -256,6 +257,48 @@ __global__ void __launch_bounds__(64 * kVecWaves) k_bgk_vec(const StepArgs a, in
   });
 
   const int self_row = D == 3 ? (w.x * a.ny + w.y) * a.nz : w.x * a.ny;
+  auto force_at = [&](int j, C* F) {
+    CellPos c;
+    c.x = w.x;
+    c.y = D == 3 ? w.y : w.k0 + j;
+    c.z = D == 3 ? w.k0 + j : 0;
+    force_of_cell<L, C>(a, c, F);
+  };
+  if constexpr (kPairs<L, S, C>) {
+    // The collision that this format's other kernels take.  Fields are stored first, so
+    // that the densities end there (D3Q19 with the exact-difference source and V = 4
+    // otherwise takes 171 registers, two wavefronts a SIMD: 96^3 45 us a step, not 38),
+    // and populations in their order (see bgk_collide_stored).
+    PairCollision<L, FS, EQ, SH, SC> cell[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      C fc[Q], F[3];
+#pragma unroll
+      for (int i = 0; i < Q; ++i) fc[i] = f[i][j];
+      force_at(j, F);
+      cell[j].set(a, fc, F);
+    }
+    if (a.store && w.active) {
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        C F[3];
+        force_at(j, F);
+        store_fields<L, C>(a, self_row + w.k0 + j, FSX, cell[j].rho, cell[j].u, F, 2.0);
+      }
+    }
+    static_for<Q>([&](auto ic) {
+      constexpr int i = decltype(ic)::value, o = opposite<L, i>();
+      C vi[V], vo[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        if constexpr (i == o) vi[j] = cell[j].rest(f[i][j]);
+        else if constexpr (i < o) cell[j].template pair<i>(f[i][j], f[o][j], vi[j], vo[j]);
+        else cell[j].template pair<o>(f[o][j], f[i][j], vo[j], vi[j]);
+      }
+      store_vec<L, i, S, C, V, SC>(a, w, self_row, voff, vi);
+    });
+    return;
+  }
   const C of = C(a.omega_f), oe = C(a.omega_eq), gc = C(a.guo_coef);
 
   // Per-cell moments and force.
@@ -275,11 +318,7 @@ __global__ void __launch_bounds__(64 * kVecWaves) k_bgk_vec(const StepArgs a, in
       moments_ref<L>(fc, rho[j], u[j], u2[j]);
       drho[j] = rho[j] - C(1);
     }
-    CellPos c;
-    c.x = w.x;
-    c.y = D == 3 ? w.y : w.k0 + j;
-    c.z = D == 3 ? w.k0 + j : 0;
-    force_of_cell<L, C>(a, c, F[j]);
+    force_at(j, F[j]);
   }
 
   if constexpr (REF) {

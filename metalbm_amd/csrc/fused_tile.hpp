@@ -14,8 +14,8 @@
 // the last step) is compiled for itself.  A lane keeps its place in the rows, so that
 // its memory offsets, its LDS neighbours and forces along y are found once.
 //
-// Rounding is that of one step at a time: every step goes through the storage type
-// and the one-step kernels' operators (the same bits in FP64; FP32 sums differ).
+// Rounding is that of one step at a time, to the bit: every step goes through the
+// storage type and the one-step kernels' collision.
 //
 // Measured, microseconds a step, one-step kernel -> this one: 128^2 FP64 4.4 -> 2.0, FP32
 // 4.5 -> 1.4 (a step of a tile is 1.3 us of dependent FP64 instructions in one

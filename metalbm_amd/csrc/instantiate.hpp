@@ -122,10 +122,10 @@ void register_combo(Registry& r, int storage, int compute) {
       // registers spill).
       constexpr bool HEAVY = std::is_same_v<C, double> && L::dimQ > 19 &&
                              (FS != SRC_ZERO || EQ != (int)EquilibriumType::TruncationMa3);
-      if constexpr (L::dimD == 3 && std::is_same_v<S, C> && !HEAVY)
+      if constexpr (L::dimD == 3 && kSeveralSteps<L, S, C> && !HEAVY)
         r.add({(int)L::Type, (int)CollisionType::BGK, FS, EQ, storage, compute, SH, 0},
               march_kernel<L, S, C, FS, EQ, SH>());
-      if constexpr (L::dimD == 2 && sizeof(S) <= sizeof(C))
+      if constexpr (L::dimD == 2 && kSeveralSteps<L, S, C>)
         r.add({(int)L::Type, (int)CollisionType::BGK, FS, EQ, storage, compute, SH, 0},
               TileKernel{{&launch_tile<L, S, C, FS, EQ, SH, 16>,
                           &launch_tile<L, S, C, FS, EQ, SH, 64>},

@@ -258,15 +258,23 @@ __device__ __forceinline__ void force_of_cell(const StepArgs& a,
   }
 }
 
-// Pull all Q populations of the cell into registers.
-template <class L, class S, class C, bool NT = false>
-__device__ __forceinline__ void pull(const StepArgs& a, const CellPos& c,
-                                     C* f) {
+// Pull all Q populations of the cell into registers: as stored, or in the compute type.
+template <class L, class S, bool NT = false>
+__device__ __forceinline__ void pull_stored(const StepArgs& a, const CellPos& c, S* f) {
   const S* __restrict__ src = static_cast<const S*>(a.src);
   static_for<L::dimQ>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
     const S* base = src + (size_t)i * (size_t)a.N;
-    f[i] = to_compute<L, i, S, C>(ld<NT>(base + pull_index<L, i>(a, c)));
+    f[i] = ld<NT>(base + pull_index<L, i>(a, c));
+  });
+}
+template <class L, class S, class C>
+__device__ __forceinline__ void pull(const StepArgs& a, const CellPos& c, C* f) {
+  S p[L::dimQ];
+  pull_stored<L, S>(a, c, p);
+  static_for<L::dimQ>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    f[i] = to_compute<L, i, S, C>(p[i]);
   });
 }
 
