@@ -68,7 +68,8 @@ enum {
                              for FP64 storage with FP32 compute, when the
                              contiguous extent (nz in 3D, ny in 2D) is
                              divisible by V; else one cell per lane (the
-                             faster shape measured for each) */
+                             faster shape measured for each).  BGK also takes
+                             several steps to a launch where that is faster */
   LBM_KERNEL_CELL = 1,    /* one cell per lane */
   LBM_KERNEL_VECTOR = 2   /* V consecutive cells per lane, aligned vector
                              accesses; needs nz (3D) / ny (2D) divisible by
@@ -176,13 +177,16 @@ const char *lbm_last_error(const lbm_handle *h);
 
 /* Sizes derived from the configuration. */
 int lbm_sizes(const lbm_handle *h, int64_t *cells, int *q, int *d);
-/* The handle's configuration (alpha_mode and residual_tol as last set;
- * kernel: the shape in use, LBM_KERNEL_CELL or LBM_KERNEL_VECTOR). */
+/* The handle's configuration (alpha_mode and residual_tol as last set; kernel
+ * as asked for, so that a handle created from it runs the same kernels;
+ * lbm_kernel_shape gives the shape that it takes). */
 int lbm_get_config(const lbm_handle *h, lbm_config *out);
 
-/* The step kernel lbm_create chooses for cfg without creating anything:
- * *shape = LBM_KERNEL_CELL or LBM_KERNEL_VECTOR and *vec = the vector
- * kernel's cells per lane V (0 for the cell kernel).  Host-only (no device
+/* The kernel of a single step that lbm_create chooses for cfg, without creating
+ * anything: *shape = LBM_KERNEL_CELL or LBM_KERNEL_VECTOR and *vec = the vector
+ * kernel's cells per lane V (0 for the cell kernel).  Asked for by that shape a
+ * handle takes every step with it; with LBM_KERNEL_AUTO, lbm_step may take several
+ * steps to a launch instead, with the same results.  Host-only (no device
  * is touched); LBM_E_INVALID for a configuration lbm_create rejects.  No
  * reference counterpart: the reference has one kernel shape
  * (Computation.cuh:39-51). */

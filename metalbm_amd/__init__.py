@@ -91,7 +91,8 @@ _QD = {LatticeType.D2Q9: (9, 2), LatticeType.D3Q19: (19, 3), LatticeType.D3Q27: 
 
 
 def kernel_shape(config: "Config"):
-    """(KernelShape, V) that lbm_create would choose for ``config``; host-only."""
+    """(KernelShape, V) of the kernel of a single step that lbm_create would choose for
+    ``config``; host-only."""
     shape, vec = ctypes.c_int(), ctypes.c_int()
     c = config.to_c()
     check(lib().lbm_kernel_shape(ctypes.byref(c), ctypes.byref(shape), ctypes.byref(vec)), None)

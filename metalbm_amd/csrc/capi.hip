@@ -685,7 +685,6 @@ int lbm_get_config(const lbm_handle* h, lbm_config* out) {
   *out = h->cfg;
   out->alpha_mode = h->alpha_mode;
   out->residual_tol = h->residual_tol;
-  out->kernel = h->vec ? LBM_KERNEL_VECTOR : LBM_KERNEL_CELL;
   return LBM_OK;
 }
 
