@@ -222,7 +222,8 @@ constexpr double kSeriesAlphaMax = 2.5;
 // Outcome of a solve from the series.
 enum : int { SOLVE_DONE = 0, SOLVE_REJECTED = 1, SOLVE_BEYOND = 2 };
 
-// Newton from the series, keeping the term-by-term solvers' results to the bit.
+// Newton from the series, keeping the term-by-term solvers' results: to the bit in FP32
+// arithmetic, their iterations and outcomes in FP64.
 //
 // Term by term, G carries rounding (gnoise, below), and so each step an error
 // up to gnoise / |G'|; the series' own is a thousand times smaller.  At tau =
@@ -231,7 +232,11 @@ enum : int { SOLVE_DONE = 0, SOLVE_REJECTED = 1, SOLVE_BEYOND = 2 };
 // change what the kernel applies or stores of alpha, or the number of
 // iterations, the cell is left to the term-by-term solver, which decides as it
 // always has (SOLVE_BEYOND; so are iterates that leave the series or are not a
-// number).  settled(x, d): whether all of [x - d, x + d] rounds to one result.
+// number).  settled(x, d): whether all of [x - d, x + d] rounds to one result.  In
+// FP64 arithmetic no alpha is settled in that sense, and the series' is taken: it
+// differs from the term-by-term one by that one's noise (4e-13 in D2Q9, 3e-14 in 3D
+// on strong noise; 1e-10 where |G'| is smallest), so that a cell's alpha depends on
+// whether its domain is large enough for the list.
 //
 // gnoise: the rounding of the 2Q quotients f / w under the logarithms, up to
 // 2^-53 (sum f + sum (f - a n)) = 2^-52 rho: 1e-10 of alpha at D2Q9 2048^2, where
