@@ -21,9 +21,9 @@ F = ForceType
 # vector kernel (0: none for this extent)
 CASES = [
     (Q19, (70, 64, 64), GUO, F.Constant, MA3, "F32", True, 4),
-    (Q19, (37, 211, 150), EDM, F.Kolmogorov, MA3, "F32", True, 2),
+    (Q19, (101, 131, 98), EDM, F.Kolmogorov, MA3, "F32", True, 2),
     (Q19, (61, 90, 101), NONE, F.None_, MA3, "F32", False, 0),
-    (Q27, (97, 90, 100), GUO, F.Sinusoidal, EXACT, "F32", True, 4),
+    (Q27, (160, 128, 100), GUO, F.Sinusoidal, EXACT, "F32", True, 4),
     (Q27, (127, 128, 126), EDM, F.Constant, EXACT, "F32", False, 2),
     (Q27, (97, 161, 129), GUO, F.Kolmogorov, EXACT, "F32", True, 0),
     (Q27, (29, 70, 530), EDM, F.Sinusoidal, MA3, "F32", True, 2),
