@@ -64,13 +64,15 @@ constexpr int opposite() {
 // (powers of two, so that the products with them, folded into the sums' and the results'
 // factors, round nothing).
 //
-// f + omega_eq (feq - f) rather than omega_f f + omega_eq feq: omega_f and omega_eq
-// rounded to single precision do not add up to 1, and that error, the same in every cell
-// and step, was most of the result's.  (EDM: omega_f (f - feq) + feq(v), for the same
-// reason.)  Error against 64 bits after 15 steps of noise on D3Q19 with tau 0.55 / 0.6624
-// / 0.8 (relative 2-norm of f - w): 5.5e-7 / 2.5e-7 / 2.0e-7; with the two rates 9.5e-7 /
-// 8.4e-7 / 2.4e-7; one population at a time, as it was before the pairs, 9.6e-7 / 6.5e-7
-// / 2.8e-7; D2Q9, 2000 steps, tau 0.53: 1.7e-5, 8.9e-5 and 9.1e-5.
+// The two rates add up to 1 exactly, the larger one in magnitude being the rounded one:
+// rounded each by itself, omega_f + omega_eq lost mass and momentum at every collision,
+// the same share in every cell, which was most of the result's error.  (EDM: omega_f (f -
+// feq) + feq(v), for which any omega_f keeps them.)  Error against 64 bits after 15 steps
+// of noise on D3Q19 with tau 0.55 / 0.6624 / 0.8 / 1.3 (relative 2-norm of f - w, Guo):
+// 6.4e-7 / 2.6e-7 / 3.0e-7 / 1.9e-7; with each rate rounded 9.9e-7 / 7.8e-7 / 3.0e-7 /
+// 3.8e-7; one population at a time, as it was before the pairs, 9.6e-7 / 6.5e-7 / 3.1e-7 /
+// 4.8e-7; D2Q9, 2000 steps, tau 0.53: 3.4e-5, 8.3e-5 and 9.1e-5.  (f + omega_eq (feq - f)
+// would give 2.2e-5 there, at 3% of the time of the 2D kernel.)
 
 // Ma3: t(cu) = base + rho (P(cu) - 1), P the polynomial (Equilibrium.h:17-33), times
 // `scale`, split into its even part e0 + cu^2 (e1 + e2 cu^2) and its odd part
@@ -123,8 +125,8 @@ struct PairCollision {
   float rho, u[3];   // the moments
   float of, oe, sum; // sum: drho (SH) or rho
   float v[3];        // EDM: u + F / rho
-  float G[3], g, uG; // Guo: omega_eq w g (c.G - u.G + 3 (c.u) (c.G)), G = F, g =
-                     // 3 (1 - 1 / (2 tau)) / omega_eq (ForcingScheme.h:99-117), uG = g u.G
+  float G[3], uG;    // Guo: w (c.G - u.G + 3 (c.u) (c.G)), G = 3 (1 - 1 / (2 tau)) F
+                     // (ForcingScheme.h:99-117)
   Ma3Split E, E2;
   ExactTerms<L> X, X2;
 
@@ -135,8 +137,10 @@ struct PairCollision {
 
   __device__ __forceinline__ void set(const StepArgs& a, const float* f, const float* F) {
     constexpr int Q = L::dimQ, D = L::dimD;
-    of = float(a.omega_f);
+    // 1 - oe is exact from 0.5 to 2, and then 1 - of from 0.5 to 1
     oe = float(a.omega_eq);
+    of = oe < 0.5f ? float(a.omega_f) : 1.0f - oe;
+    oe = oe < 0.5f ? 1.0f - of : oe;
     sum = f[0] * (1.0f / scale_of<0>());
     float j[3] = {0.0f, 0.0f, 0.0f};
     static_for<Q>([&](auto ic) {
@@ -153,26 +157,24 @@ struct PairCollision {
       }
     });
     rho = SH ? 1.0f + sum : sum;
-    // The reciprocal estimate with one correction, and each quotient's remainder
-    // through it: a biased 1 / rho biases every equilibrium velocity (see
-    // moments_shifted_scaled).
     const float r0 = __builtin_amdgcn_rcpf(rho);
-    const float rr = fmaf(r0, fmaf(-rho, r0, 1.0f), r0);
+    const float rr = fmaf(r0, fmaf(-rho, r0, 1.0f), r0);  // see moments_shifted_scaled
     u[2] = v[2] = 0.0f;
     for (int d = 0; d < D; ++d) {
-      const float q = j[d] * rr;
-      u[d] = fmaf(rr, fmaf(-rho, q, j[d]), q);
+      u[d] = j[d] * rr;
+      asm("" : "+v"(u[d]));  // no longer a product: c.u adds them
     }
     if constexpr (FS == SRC_EDM)  // feq(rho, u + F / rho) - feq (ForcingScheme.h:184-197)
       for (int d = 0; d < D; ++d) v[d] = fmaf(F[d], rr, u[d]);
     uG = 0.0f;
     if constexpr (FS == SRC_GUO) {
-      g = float(3.0 * a.guo_coef / a.omega_eq);
-      // summed by itself: taken from E.e0 term by term, its roundings moved the mean
+      const float g = float(3.0 * a.guo_coef);
+      // uG summed by itself: taken from E.e0 term by term, its roundings moved the mean
       // density by 1e-12 a step, always one way
       for (int d = 0; d < D; ++d) {
-        G[d] = F[d];
-        uG = fmaf(u[d], g * F[d], uG);
+        G[d] = g * F[d];
+        asm("" : "+v"(G[d]));  // likewise
+        uG = fmaf(u[d], G[d], uG);
       }
     }
     if constexpr (MA3) {
@@ -181,7 +183,7 @@ struct PairCollision {
         for (int d = 1; d < D; ++d) s = fmaf(w[d], w[d], s);
         return s;
       };
-      E.set(FS == SRC_EDM ? -of : 1.0f, rho, sum, square(u));
+      E.set(FS == SRC_EDM ? -of : oe, rho, sum, square(u));
       if constexpr (FS == SRC_GUO) E.e0 -= uG;
       if constexpr (FS == SRC_EDM) {
         E2.set(1.0f, rho, sum, square(v));
@@ -193,25 +195,20 @@ struct PairCollision {
     }
   }
 
-  // Post-collision from the pulled f and t: feq / w - (SH ? 1 : 0) with the source (EDM:
-  // feq(v) / w ... - omega_f feq / w ...).
-  __device__ __forceinline__ float relaxed(float w, float t, float f) const {
-    if constexpr (FS == SRC_EDM) return fmaf(w, t, of * f);
-    else return fmaf(oe, fmaf(w, t, -f), f);
-  }
-  // t of the product equilibrium, without Guo's source.
+  // Product equilibrium: omega_eq feq_i / w_i (less omega_eq if SH) and the source over
+  // w_i, for EDM -omega_f feq_i(u) / w_i + feq_i(v) / w_i.
   template <int i>
-  __device__ __forceinline__ float exact() const {
+  __device__ __forceinline__ float exact(float source) const {
     const float t = fmaf(rho, X.template p<i>(), sum);
     if constexpr (FS == SRC_EDM) return fmaf(-of, t, fmaf(rho, X2.template p<i>(), sum));
-    else return t;
+    else return fmaf(oe, t, source);
   }
 
-  // Population 0 and the pair i, opposite<L, i>().
+  // Population 0 and the pair i, opposite<L, i>(): pulled to post-collision.
   __device__ __forceinline__ float rest(float f) const {
     constexpr float w = float(L::W[0]) * scale_of<0>();
-    if constexpr (MA3) return relaxed(w, E.e0, f);
-    else return relaxed(w, FS == SRC_GUO ? exact<0>() - uG : exact<0>(), f);
+    if constexpr (MA3) return fmaf(w, E.e0, of * f);
+    else return fmaf(w, exact<0>(-uG), of * f);
   }
   template <int i>
   __device__ __forceinline__ void pair(float fi, float fo, float& to_i, float& to_o) const {
@@ -219,7 +216,7 @@ struct PairCollision {
     constexpr float w = float(L::W[i]) * scale_of<i>();
     const float cu = cdot<L, i>(u);
     float cG = 0.0f;
-    if constexpr (FS == SRC_GUO) cG = cdot<L, i>(G);  // of loaded values: no products
+    if constexpr (FS == SRC_GUO) cG = cdot<L, i>(G);
     float ti, to;
     if constexpr (MA3) {
       const float q = cu * cu;
@@ -231,8 +228,8 @@ struct PairCollision {
       } else {
         float odd;
         if constexpr (FS == SRC_GUO) {
-          even = fmaf(3.0f * cu, g * cG, even);
-          odd = fmaf(cu, E.odd(q), g * cG);
+          even = fmaf(3.0f * cu, cG, even);
+          odd = fmaf(cu, E.odd(q), cG);
         } else {
           const float cv = cdot<L, i>(v), r = cv * cv;
           even = E2.even(r, even);
@@ -241,17 +238,16 @@ struct PairCollision {
         ti = even + odd;
         to = even - odd;
       }
+    } else if constexpr (FS == SRC_GUO) {
+      const float even = fmaf(3.0f * cu, cG, -uG);
+      ti = exact<i>(even + cG);
+      to = exact<o>(even - cG);
     } else {
-      ti = exact<i>();
-      to = exact<o>();
-      if constexpr (FS == SRC_GUO) {
-        const float even = fmaf(3.0f * cu, g * cG, -uG);
-        ti += fmaf(g, cG, even);
-        to += fmaf(-g, cG, even);
-      }
+      ti = exact<i>(0.0f);
+      to = exact<o>(0.0f);
     }
-    to_i = relaxed(w, ti, fi);
-    to_o = relaxed(w, to, fo);
+    to_i = fmaf(w, ti, of * fi);
+    to_o = fmaf(w, to, of * fo);
   }
 };
 
@@ -356,6 +352,8 @@ __device__ __forceinline__ void bgk_collide_stored(const StepArgs& a, const S* p
   static_for<L::dimQ>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
     f[i] = SC ? C(p[i]) : to_compute<L, i, S, C>(p[i]);
+    // converted once, not again in each operation (mixed-precision ones are slower)
+    if constexpr (SC) asm("" : "+v"(f[i]));
   });
   auto stored = [&](auto ic, C v) {
     constexpr int i = decltype(ic)::value;
