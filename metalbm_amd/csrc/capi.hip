@@ -306,15 +306,15 @@ int ensure_fields(lbm_handle* h) {
 // way while it copies the other (35 MB, ten steps of D3Q19 96 x 80 x 72 and the copy:
 // 3.41 -> 1.70 ms; 94 MB: 9.8 -> 4.1; 12 MB: 0.90 -> 0.63).  Requests of fewer bytes
 // than the pinned memory, and pinned or device destinations, are copied directly.
-// The calling thread waits for the handle's stream before the others start, and the
-// chunks go through a stream of their own: a handle's stream may be hipStreamPerThread,
-// which is another stream in each thread.
+// The calling thread waits for the handle's stream before the others start, and each
+// thread for its own copies: a handle's stream may be hipStreamPerThread, which is
+// another stream in each thread.
 struct FieldPart {
   char* dst;
   const char* src;
   size_t bytes;
 };
-// Pinned chunks, two to a copying thread, with their events and stream.  A process
+// Pinned chunks, two to a copying thread, with their events.  A process
 // has at most kRings of them, whichever handles use them (a call that finds all in
 // use copies directly), and frees them with its last handle.
 constexpr int kRingSlots = 8, kRings = 4;
@@ -322,7 +322,6 @@ constexpr size_t kRingChunk = 1 << 20;
 struct FieldRing {
   int device = -1;
   char* mem = nullptr;
-  hipStream_t stream = nullptr;
   hipEvent_t event[kRingSlots] = {};
 };
 struct RingPool {
@@ -335,7 +334,6 @@ RingPool g_rings;
 void free_ring(FieldRing* r) {
   for (hipEvent_t e : r->event)
     if (e) (void)hipEventDestroy(e);
-  if (r->stream) (void)hipStreamDestroy(r->stream);
   if (r->mem) (void)hipHostFree(r->mem);
   delete r;
 }
@@ -361,7 +359,6 @@ FieldRing* take_ring(int device) {
   if (other) free_ring(other);
   FieldRing* r = new (std::nothrow) FieldRing;
   bool ok = r && hipHostMalloc(&r->mem, kRingSlots * kRingChunk, hipHostMallocDefault) == hipSuccess;
-  ok = ok && hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking) == hipSuccess;
   for (int k = 0; ok && k < kRingSlots; ++k)
     ok = hipEventCreateWithFlags(&r->event[k], hipEventDisableTiming) == hipSuccess;
   if (ok) {
@@ -416,8 +413,8 @@ hipError_t copy_through_ring(lbm_handle* h, FieldRing& ring, const FieldPart* pa
       if (error != hipSuccess || !chunk(next++, &c[k])) return false;
       const int slot = 2 * w + k;
       hipError_t e = hipMemcpyAsync(ring.mem + slot * kRingChunk, c[k].src, c[k].bytes,
-                                    hipMemcpyDeviceToHost, ring.stream);
-      if (e == hipSuccess) e = hipEventRecord(ring.event[slot], ring.stream);
+                                    hipMemcpyDeviceToHost, h->stream);
+      if (e == hipSuccess) e = hipEventRecord(ring.event[slot], h->stream);
       if (e != hipSuccess) error = e;
       return e == hipSuccess;
     };
@@ -433,6 +430,8 @@ hipError_t copy_through_ring(lbm_handle* h, FieldRing& ring, const FieldPart* pa
       }
       std::memcpy(c[k].dst, ring.mem + slot * kRingChunk, c[k].bytes);
     }
+    // every copy of this thread has been waited for, unless one failed
+    if (error != hipSuccess) (void)hipStreamSynchronize(h->stream);
   };
   std::thread helpers[kRingSlots / 2];
   for (int w = 1; w < kRingSlots / 2; ++w) {
@@ -445,9 +444,7 @@ hipError_t copy_through_ring(lbm_handle* h, FieldRing& ring, const FieldPart* pa
   work(0);
   for (auto& t : helpers)
     if (t.joinable()) t.join();
-  // every chunk has been waited for, unless one failed
-  const hipError_t e = hipStreamSynchronize(ring.stream);
-  return error != hipSuccess ? (hipError_t)error.load() : e;
+  return (hipError_t)error.load();
 }
 
 // State every initialiser starts from.  The entropic alpha field restarts at
