@@ -1126,17 +1126,14 @@ int lbm_step(lbm_handle* h, int nsteps, int store_last) {
   // step.
   int paired = h->march ? (nsteps - (store_last ? 1 : 0)) / 4 * 4 : 0;
   // The 2D kernel stores as well; as many launches, modulo two, as steps.
-  int launches = nsteps;
-  if (h->tile && nsteps > 1) {
-    launches = (nsteps + h->tile2d.steps - 1) / h->tile2d.steps;
-    launches += (nsteps - launches) & 1;
-  }
+  int launches = h->tile ? launches_of(nsteps, h->tile2d.steps) : nsteps;
   for (int s = 0, n = 1; s < nsteps; s += n) {
     if (paired > 0) {
       n = 2;
       paired -= 2;
     } else if (h->tile) {
-      n = (nsteps - s + launches - 1) / launches--;
+      n = steps_of_next(nsteps - s, launches);
+      --launches;
     } else {
       n = 1;
     }

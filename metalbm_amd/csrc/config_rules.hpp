@@ -306,4 +306,15 @@ inline TileShape tile_shape(int nx, int ny, const int (&rows)[2], bool fp64, boo
   return best;
 }
 
+// Launches of at most `per` steps each for `steps` steps: as many, modulo two, as steps,
+// so that the populations end in the lattice that one launch a step would leave them in.
+inline int launches_of(int steps, int per) {
+  const int n = steps / per + (steps % per != 0);
+  return n + ((steps - n) & 1);
+}
+// Steps of the next of `launches` launches with `steps` left.
+inline int steps_of_next(int steps, int launches) {
+  return steps / launches + (steps % launches != 0);
+}
+
 }  // namespace lbm
