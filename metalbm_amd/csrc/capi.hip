@@ -502,9 +502,8 @@ bool certified_mode(const lbm_handle* h) {
 
 // Whether a step lists cells for a second launch (see k_elbm): the certified
 // modes always; on larger domains the Newton modes in 3D and the reference
-// Newton in D2Q9, where the list exists (it is allocated with the handle or when
-// such a mode is set; without the memory for it the term-by-term kernels solve
-// every cell).  The parity build's reference Newton never does.
+// Newton in D2Q9, where the list exists (without the memory for it the term-by-term
+// kernels solve every cell).  The parity build's reference Newton never does.
 bool newton_lists(const lbm_handle* h) {
   const bool parity = h->ctype == TYPE_F64 && !h->cfg.shifted;
   if (certified_mode(h) || (h->alpha_mode == LBM_ALPHA_NEWTON && parity)) return false;
@@ -537,9 +536,17 @@ hipError_t allocate_list(lbm_handle* h) {
   return e;
 }
 
-// For a Newton mode that lists cells, if there is room (see lists_cells).
-void allocate_newton_list(lbm_handle* h) {
-  if (newton_lists(h) && allocate_list(h) != hipSuccess) (void)hipGetLastError();
+// With the handle, and when a mode is set that lists cells, so that a call's first steps
+// can be captured in a graph (an allocation ends a capture).  Without the memory a Newton
+// mode goes on term by term, and a certified mode's lbm_step tries again and reports it.
+void prepare_list(lbm_handle* h) {
+  if (!certified_mode(h) && !newton_lists(h)) return;
+  int current = -1;
+  if (hipGetDevice(&current) == hipSuccess &&
+      (current == h->device || hipSetDevice(h->device) == hipSuccess))
+    (void)allocate_list(h);
+  if (current >= 0 && current != h->device) (void)hipSetDevice(current);
+  if (!h->defer_list) (void)hipGetLastError();
 }
 
 StepArgs make_args(const lbm_handle* h) {
@@ -787,7 +794,7 @@ int lbm_create(const lbm_config* cfg, lbm_handle** out) {
       h->err = std::string("alpha field: ") + hipGetErrorString(e);
       return bail(LBM_E_HIP);
     }
-    allocate_newton_list(h);
+    prepare_list(h);
   }
   *out = h;
   count_handle(1);
@@ -1787,7 +1794,7 @@ int lbm_set_alpha_mode(lbm_handle* h, int mode, double residual_tol) {
     return fail(h, LBM_E_INVALID, "residual_tol must be positive");
   h->alpha_mode = mode;
   if (residual_tol > 0.0) h->residual_tol = residual_tol;
-  allocate_newton_list(h);
+  prepare_list(h);
   return LBM_OK;
 }
 
