@@ -206,6 +206,32 @@ __device__ __forceinline__ void store_vec(const StepArgs& a, const WavePos& w,
               make_rsrc(row, (unsigned)a.nk * (unsigned)sizeof(S)), voff, 0);
 }
 
+// store_fields for a lane's V cells in single precision, field by field: a cell at a time,
+// the V parts of a line are written far apart, with loads of the force between them that
+// wait for the earlier stores (storing steps, V = 4: D2Q9 2048^2 177 us, 98 so; D3Q19
+// 192^3 441 and 316).
+template <class L, int V>
+__device__ __forceinline__ void store_fields_row(const StepArgs& a, int cell, int FS,
+                                                 const float (&rho)[V], const float (&u)[V][3],
+                                                 const float (&F)[V][3]) {
+  auto store = [&](double* field, auto&& value) {
+#pragma unroll
+    for (int j = 0; j < V; ++j) field[cell + j] = double(value(j));
+  };
+  store(a.rho_out, [&](int j) { return rho[j]; });
+  float h[V];  // see store_fields
+#pragma unroll
+  for (int j = 0; j < V; ++j) h[j] = FS == (int)ForcingSchemeType::None ? 0.0f : 0.5f / rho[j];
+  for (int d = 0; d < L::dimD; ++d)
+    store(a.uh_out + (size_t)d * a.N, [&](int j) {
+      return FS == (int)ForcingSchemeType::None ? u[j][d] : fmaf(F[j][d], h[j], u[j][d]);
+    });
+  if (a.alpha_out) store(a.alpha_out, [](int) { return 2.0; });
+  if (a.F_out)
+    for (int d = 0; d < L::dimD; ++d)
+      store(a.F_out + (size_t)d * a.N, [&](int j) { return F[j][d]; });
+}
+
 template <class L, class S, class C, int FS, int EQ, bool SH, int V>
 __global__ void __launch_bounds__(64 * kVecWaves) k_bgk_vec(const StepArgs a, int FSX) {
   constexpr int Q = L::dimQ, D = L::dimD;
@@ -268,7 +294,10 @@ __global__ void __launch_bounds__(64 * kVecWaves) k_bgk_vec(const StepArgs a, in
     // The collision that this format's other kernels take.  Fields are stored first, so
     // that the densities end there (D3Q19 with the exact-difference source and V = 4
     // otherwise takes 171 registers, two wavefronts a SIMD: 96^3 45 us a step, not 38),
-    // and populations in their order (see bgk_collide_stored).
+    // and populations in their order, each pair's second one waiting in the register of
+    // the pulled one (the empty asm statement: left alone, the compiler forms it where it
+    // is stored and holds the pair's terms instead, 211 registers for 156 in D3Q27
+    // without a source and V = 4: 96^3 66 us a step for 53).
     PairCollision<L, FS, EQ, SH, SC> cell[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) {
@@ -279,23 +308,26 @@ __global__ void __launch_bounds__(64 * kVecWaves) k_bgk_vec(const StepArgs a, in
       cell[j].set(a, fc, F);
     }
     if (a.store && w.active) {
+      C rho[V], u[V][3], F[V][3];
 #pragma unroll
       for (int j = 0; j < V; ++j) {
-        C F[3];
-        force_at(j, F);
-        store_fields<L, C>(a, self_row + w.k0 + j, FSX, cell[j].rho, cell[j].u, F, 2.0);
+        rho[j] = cell[j].rho;
+        for (int d = 0; d < 3; ++d) u[j][d] = cell[j].u[d];
+        force_at(j, F[j]);
       }
+      store_fields_row<L, V>(a, self_row + w.k0, FSX, rho, u, F);
     }
     static_for<Q>([&](auto ic) {
       constexpr int i = decltype(ic)::value, o = opposite<L, i>();
-      C vi[V], vo[V];
 #pragma unroll
       for (int j = 0; j < V; ++j) {
-        if constexpr (i == o) vi[j] = cell[j].rest(f[i][j]);
-        else if constexpr (i < o) cell[j].template pair<i>(f[i][j], f[o][j], vi[j], vo[j]);
-        else cell[j].template pair<o>(f[o][j], f[i][j], vo[j], vi[j]);
+        if constexpr (i == o) f[i][j] = cell[j].rest(f[i][j]);
+        else if constexpr (i < o) {
+          cell[j].template pair<i>(f[i][j], f[o][j], f[i][j], f[o][j]);
+          asm volatile("" : "+v"(f[o][j]));
+        }
       }
-      store_vec<L, i, S, C, V, SC>(a, w, self_row, voff, vi);
+      store_vec<L, i, S, C, V, SC>(a, w, self_row, voff, f[i]);
     });
     return;
   }
