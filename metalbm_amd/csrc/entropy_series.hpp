@@ -302,45 +302,34 @@ __device__ __forceinline__ int series_newton_residual(const SERIES& s, double st
 // whose Taylor remainder bound is <= tol without evaluating G there: G(a1) =
 // s^2/2 G''(xi) for some xi between a and a1, and f - xi n = (f - a n) +
 // (a - xi) n >= (f - a n)(1 - |s| r), so |G''(xi)| <= h / (1 - |s| r); a relative
-// allowance of 1e-6 covers the rounding of the bound.  Anything else is left
-// to plain Newton from the stored alpha (SOLVE_REJECTED).
-//
-// OWN: `start` is the stored alpha, so the iterates are plain Newton's own; they are
-// accepted where series_newton_residual would accept them (its thresholds, its
-// settled), so that the result is plain Newton's to the bit.
-template <bool OWN, class SERIES, class SETTLED>
-__device__ __forceinline__ int series_correction(const SERIES& s, double start, double tol,
-                                                 int max_evals, double gnoise, double& alpha,
-                                                 int& evals, EvalCurv& cv, SETTLED&& settled) {
-  double a = start, before = 0.0;
+// allowance of 1e-6 covers the rounding of the bound.  Anything else defers
+// the cell to plain Newton from the stored alpha.
+template <class SERIES>
+__device__ __forceinline__ bool series_correction(const SERIES& s, double start,
+                                                  double tol, int max_evals, double& alpha,
+                                                  int& evals, EvalCurv& cv) {
+  double a = start;
   for (int it = 0; it < max_evals; ++it) {
-    if (!(a > 1.0 && a < kSeriesAlphaMax) || !s.holds(a)) return SOLVE_REJECTED;
+    if (!(a > 1.0 && a < kSeriesAlphaMax) || !s.holds(a)) return false;
     double g, dg;
     s.eval(a, g, dg);
     cv = s.curvature(a, dg);
     evals = it + 1;
-    const double noise = OWN ? fabs(gnoise / dg) : 0.0;
-    if (OWN && !(fabs(fabs(g) - tol) > gnoise + before * fabs(dg))) return SOLVE_BEYOND;
     if (fabs(g) <= tol) {
-      if (OWN && !settled(a, before)) return SOLVE_BEYOND;
       alpha = a;
-      return SOLVE_DONE;
+      return true;
     }
     const double step = g / dg;
     const double a1 = a - step;
     const double room = 1.0 - fabs(step) * cv.r;
-    // at a1 plain Newton would find |G| <= tol by more than the noise of the two sides
-    const double within = OWN ? tol - 3.0 * gnoise : tol;
     if (a1 > 1.0 && a1 < kSeriesAlphaMax && room > 0.0 &&
-        0.5 * step * step * cv.h / room * (1.0 + 1e-6) <= within) {
-      if (OWN && !settled(a1, noise)) return SOLVE_BEYOND;
+        0.5 * step * step * cv.h / room * (1.0 + 1e-6) <= tol) {
       alpha = a1;
-      return SOLVE_DONE;
+      return true;
     }
     a = a1;
-    before = noise;
   }
-  return SOLVE_REJECTED;
+  return false;
 }
 
 // Runs body(series) with the shortest series that holds for every active lane

@@ -893,18 +893,16 @@ __global__ void __launch_bounds__(BLOCK)
             outcome = series_newton_reference(s, stored, gnoise, alpha, its, settled);
           } else {
             int before = 0;
-            outcome = SOLVE_REJECTED;
             if constexpr (MODE != 4) {
               EvalCurv cv{};
-              outcome = series_correction<MODE == 2>(s, MODE == 1 ? start : stored,
-                                                     a.residual_tol, MODE == 1 ? 1 : 2, gnoise,
-                                                     alpha, before, cv, settled);
-              if (MODE == 1 && outcome == SOLVE_DONE &&
-                  !reference_reaches(cv, alpha, stored, a.residual_tol))
-                outcome = SOLVE_REJECTED;
-              first = outcome == SOLVE_DONE;
+              first = series_correction(s, MODE == 1 ? start : stored, a.residual_tol,
+                                        MODE == 1 ? 1 : 2, alpha, before, cv);
+              if constexpr (MODE == 1)
+                first = first && reference_reaches(cv, alpha, stored, a.residual_tol);
             }
-            if (outcome == SOLVE_REJECTED)
+            if (first)
+              outcome = SOLVE_DONE;
+            else
               outcome = series_newton_residual(s, stored, a.residual_tol, gnoise, alpha, its,
                                                settled);
             its += before;
