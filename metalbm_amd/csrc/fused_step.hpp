@@ -717,16 +717,22 @@ __device__ __forceinline__ unsigned sample_hash(unsigned cell, unsigned salt) {
 template <int MODE>
 constexpr bool kListMode = MODE == 3 || MODE == 5 || MODE == 7;
 
-// Minimum wavefronts per SIMD the register allocator must leave room for.
-template <class L, int MODE>
+// Minimum wavefronts per SIMD the register allocator must leave room for: the FP64 solve
+// waits for its own results, so three gain over two where they spill little (FP32
+// arithmetic up to 25 registers, D3Q19 in FP64 up to 60).  Two where three spilled more:
+// D3Q27 in FP64 arithmetic (41 to 183; plain Newton 24^3 37 -> 22 us, 96 x 90 x 100 near
+// equilibrium 228 -> 152, stored alpha 180 -> 147), and MODE 7 (FP32 64^3 with strong
+// noise 83 -> 71, D3Q19 FP64 32^3 23 -> 17).
+template <class L, class C, int MODE>
 constexpr int elbm_min_waves() {
   if (L::Type == LatticeType::D2Q9) return kListMode<MODE> || MODE == 6 ? 2 : 4;
-  return MODE == 6 ? 2 : 3;
+  if (std::is_same_v<C, double> && L::dimQ > 19) return 2;
+  return MODE == 6 || MODE == 7 ? 2 : 3;
 }
 
 template <class L, class S, class C, int FS, int EQ, bool SH, int BLOCK, int MODE>
 __global__ void __launch_bounds__(BLOCK)
-    __attribute__((amdgpu_waves_per_eu(elbm_min_waves<L, MODE>())))
+    __attribute__((amdgpu_waves_per_eu(elbm_min_waves<L, C, MODE>())))
     k_elbm(const StepArgs a, int FSX) {
   constexpr int Q = L::dimQ;
   constexpr bool REF = std::is_same_v<C, double> && !SH;
