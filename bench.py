@@ -101,7 +101,8 @@ WORKLOADS = {
         init=("noise", 1e-3, 42), steps=200),
     "d3q27-elbm-256-newton-residual": dict(
         desc="D3Q27 SRT Entropic 256^3 as d3q27-elbm-256-newton, plain Newton at the "
-             "residual tolerance: from the stored alpha until |G| <= 1e-10, one launch",
+             "residual tolerance: from the stored alpha until |G| <= 1e-10, the cells that "
+             "its power sums do not settle in a second launch",
         cfg=dict(lattice="D3Q27", collision="ELBM", nx=256, ny=256, nz=256, tau=0.50006,
                  forcing_scheme="None_", force="None_", storage="F32", compute="F32",
                  shifted=True, alpha_mode="NEWTON_RESIDUAL", residual_tol=1e-10),
