@@ -304,8 +304,9 @@ int ensure_fields(lbm_handle* h) {
 // pages, most of them touched for the first time: 12 GB/s of the link's 54.  Here the
 // chunks go to pinned memory and four threads empty it, each with one chunk on its
 // way while it copies the other (35 MB, ten steps of D3Q19 96 x 80 x 72 and the copy:
-// 3.41 -> 1.70 ms; 94 MB: 9.8 -> 4.1; 12 MB: 0.90 -> 0.63).  Requests of fewer bytes
-// than the pinned memory, and pinned or device destinations, are copied directly.
+// 2.5 -> 1.6 ms; where the host's pages came slower 4.1 -> 1.8, 94 MB 9.4 -> 4.2, 12 MB
+// 2.2 -> 0.6).  Requests of fewer bytes than the pinned memory, and pinned or device
+// destinations, are copied directly.
 // The calling thread waits for the handle's stream before the others start, and each
 // thread for its own copies: a handle's stream may be hipStreamPerThread, which is
 // another stream in each thread.

@@ -28,11 +28,11 @@
 // others collide.  (All four columns in flight: the compiler spills 20 registers
 // of loads not yet there, whose waits cost a third of the time.)
 //
-// Measured, microseconds a step, one-step kernels -> this one: D3Q19 256^3 456 ->
-// 257 (1.46 GB read and 1.28 GB written by a launch of 513 us, 5.3 TB/s; 64 % of
-// the vector issue slots), D3Q27 193 x 161 x 130 Ma3 260 -> 159, product
-// equilibrium 276 -> 183; FP64, one column a thread: D3Q19 192^3 424 -> 328, 171 x
-// 150 x 133 257 -> 208 (60 % of the issue slots: before opposite populations shared
+// Measured, microseconds a step, one-step kernels -> this one: D3Q19 256^3 461 ->
+// 257 (1.45 GB read and 1.28 GB written by a launch of 513 us, 5.3 TB/s; 64 % of
+// the vector issue slots), D3Q27 193 x 161 x 130 Ma3 290 -> 129, product
+// equilibrium 282 -> 152; FP64, one column a thread: D3Q19 192^3 422 -> 321, 171 x
+// 150 x 133 257 -> 207 (60 % of the issue slots: before opposite populations shared
 // their terms 246, with divisions by 6 and 24 304).  FP16 (D3Q27 384^3, waiting
 // populations packed in pairs: 1162 against 1205, 72 % of the issue slots at half the
 // bytes, but 192^3 1.01 to 1.21 and 64^3 2.2 times the one-step kernel's time) stays

@@ -54,7 +54,7 @@ constexpr int opposite() {
 // The single-precision BGK collision of one cell (Collision.h:134-151), two opposite
 // populations at a time: they share every term of the Ma3 equilibrium and of the
 // source up to the sign of the odd part (the two-step kernel on D3Q19 256^3 with the
-// Guo source: 179 million vector instructions a launch instead of 248, addresses
+// Guo source: 172 million vector instructions a launch instead of 248, addresses
 // included).  Every kernel that one handle's steps may go through takes its arithmetic
 // from here, so that a result does not depend on how steps are split over launches and
 // calls.  For that each kernel has to round the same way, and the compiler, which in
@@ -705,7 +705,8 @@ __device__ __forceinline__ unsigned sample_hash(unsigned cell, unsigned salt) {
 // reference Newton D2Q9 2048^2 474 -> 190 us, D3Q27 256^3 5.75 -> 1.70 ms; plain
 // Newton D3Q27 4.83 -> 1.65 ms, stored-alpha correction D3Q27 4.23 -> 1.70 ms.
 // D2Q9's other modes take one or two evaluations in the log1p form already,
-// most of what the power sums cost (147-167 us of 153), and stay.
+// most of what the power sums cost (plain Newton 173 us, the corrections 134 and 181 of
+// which the network's inference is 47), and stay.
 // Three phases so that the learned mode's wavefront-wide matrix-core
 // inference runs with every lane present: (1) pull, moments, fneq and the
 // deviation test per cell; (2) MODE 1 only: the network predicts alpha for

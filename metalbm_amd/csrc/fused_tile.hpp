@@ -1,6 +1,6 @@
 // fused_tile.hpp -- several BGK steps of a 2D lattice in one launch.
 //
-// A step of a small lattice is a launch and little else (D2Q9 128^2: 4.4 us a step,
+// A step of a small lattice is a launch and little else (D2Q9 128^2: 3.4 us a step,
 // 2.5 of them the launch), and one of a large lattice runs at what the memory streams
 // (2048^2 FP32: 55 us).  A workgroup takes a tile with a halo through several steps
 // in LDS: the first one pulls from memory, the halo shrinks by a cell a step, and the
@@ -17,11 +17,12 @@
 // Rounding is that of one step at a time, to the bit: every step goes through the
 // storage type and the one-step kernels' collision.
 //
-// Measured, microseconds a step, one-step kernel -> this one: 128^2 FP64 4.4 -> 2.0, FP32
-// 4.5 -> 1.4 (a step of a tile is 1.3 us of dependent FP64 instructions in one
-// wavefront a SIMD); 2048^2 FP32 55 -> 23, FP64 113 -> 82, FP16 38 -> 21: bound by the
-// vector instructions (five steps with a force field in FP32, 164 us: 80 % of the issue
-// slots, a quarter of the work in halos; with the parities chosen at run time 184 us).
+// Measured, microseconds a step, one-step kernel -> this one: 128^2 FP64 3.4 -> 1.8, FP32
+// and FP16 3.7 -> 1.2 (one handle, a hundred steps a call: launch, load and the dependent
+// instructions of one wavefront a SIMD; four handles on streams of their own overlap, 1.1
+// and 0.6 each); 2048^2 FP32 55 -> 22, FP64 113 -> 74, FP16 34 -> 21: bound by the vector
+// instructions (five steps with a force field in FP32, 149 us: 87 % of the issue slots, a
+// quarter of the work in halos; with the parities chosen at run time it took 12 % longer).
 #pragma once
 
 #include "fused_step.hpp"

@@ -2,9 +2,9 @@
 //
 // No reference counterpart: the reference finds alpha by Newton only
 // (Collision.h:328-349).  Here a small ReLU MLP maps the cell's normalised
-// non-equilibrium moments to a first guess of alpha; series_correction
-// (entropy_series.hpp) then certifies or corrects it, and plain Newton from
-// the stored alpha takes over when it cannot.
+// non-equilibrium moments to a first guess of alpha; residual_correction (D2Q9,
+// below) or series_correction (3D, entropy_series.hpp) then certifies or corrects
+// it, and plain Newton from the stored alpha takes over when it cannot.
 //
 // Features: m_k = (1/rho) sum_i fneq_i prod_d phi_{a_kd}(c_id), phi_0 = 1,
 // phi_1 = c, phi_2 = c^2, over the full tensor basis a_k in {0,1,2}^D (the
