@@ -94,17 +94,19 @@ struct Ma3Split {
 };
 
 // Product equilibrium: ExactShifted's factors e[d][c + 1] = phi_d^c - 1 with its fused
-// operations written out.
+// operations written out, and s = sqrt(1 + 3 v^2) taken as 1 + sm1 throughout: half of the
+// square roots just above 1 lie just below the middle of two floats and round down, which
+// shows in the momentum (1e-8 of it a collision).
 template <class L>
 struct ExactTerms {
   float e[3][3];
   __device__ __forceinline__ void set(const float* u) {
     for (int d = 0; d < L::dimD; ++d) {
       const float v = u[d], t = 3.0f * v;
-      const float s = sqrtf(fmaf(t, v, 1.0f)), sm1 = (t * v) / (1.0f + s);
+      const float sm1 = (t * v) / (1.0f + sqrtf(fmaf(t, v, 1.0f)));
       e[d][1] = -sm1;
-      e[d][2] = fmaf(v, fmaf(-2.0f, s, 5.0f), fmaf(2.0f, sm1, -(t * v))) / (1.0f - v);
-      e[d][0] = fmaf(v, s, fmaf(-4.0f, v, -2.0f * sm1)) / fmaf(2.0f, v, s);
+      e[d][2] = fmaf(v, fmaf(-2.0f, sm1, 3.0f), fmaf(2.0f, sm1, -(t * v))) / (1.0f - v);
+      e[d][0] = fmaf(v, sm1, fmaf(-3.0f, v, -2.0f * sm1)) / (fmaf(2.0f, v, 1.0f) + sm1);
     }
   }
   template <int i>
@@ -162,6 +164,9 @@ struct PairCollision {
     u[2] = v[2] = 0.0f;
     for (int d = 0; d < D; ++d) {
       u[d] = j[d] * rr;
+      // 1 / rho of a density below 1 rounds up more often than down: the quotient itself
+      // (the polynomial's error has room for it, see above)
+      if constexpr (!MA3) u[d] = fmaf(fmaf(-rho, u[d], j[d]), rr, u[d]);
       asm("" : "+v"(u[d]));  // no longer a product: c.u adds them
     }
     if constexpr (FS == SRC_EDM)  // feq(rho, u + F / rho) - feq (ForcingScheme.h:184-197)
