@@ -67,12 +67,13 @@ constexpr int opposite() {
 // The two rates add up to 1 exactly, the larger one in magnitude being the rounded one:
 // rounded each by itself, omega_f + omega_eq lost mass and momentum at every collision,
 // the same share in every cell, which was most of the result's error.  (EDM: omega_f (f -
-// feq) + feq(v), for which any omega_f keeps them.)  Error against 64 bits after 15 steps
-// of noise on D3Q19 with tau 0.55 / 0.6624 / 0.8 / 1.3 (relative 2-norm of f - w, Guo):
-// 6.4e-7 / 2.6e-7 / 3.0e-7 / 1.9e-7; with each rate rounded 9.9e-7 / 7.8e-7 / 3.0e-7 /
-// 3.8e-7; one population at a time, as it was before the pairs, 9.6e-7 / 6.5e-7 / 3.1e-7 /
-// 4.8e-7; D2Q9, 2000 steps, tau 0.53: 3.4e-5, 8.3e-5 and 9.1e-5.  (f + omega_eq (feq - f)
-// would give 2.2e-5 there, at 3% of the time of the 2D kernel.)
+// feq) + feq(v), for which any omega_f keeps them.)  The velocity is the rounded quotient
+// (two operations a component: 0.2% of the 3D kernel's time, 1% of the 2D one's).  Error
+// against 64 bits after 15 steps of noise on D3Q19 64^3 with tau 0.55 / 0.6624 / 0.8 / 1.3
+// (relative 2-norm of f - w, Guo): 6.0e-7 / 2.7e-7 / 2.7e-7 / 1.5e-7; with each rate rounded
+// and the product with 1 / rho 10e-7 / 6.8e-7 / 4.3e-7 / 4.4e-7; one population at a time,
+// as it was before the pairs, 9.9e-7 / 5.2e-7 / 4.7e-7 / 5.1e-7; D2Q9 96^2, 2000 steps, tau
+// 0.53: 2.8e-5, 8.3e-5 and 7.4e-5.
 
 // Ma3: t(cu) = base + rho (P(cu) - 1), P the polynomial (Equilibrium.h:17-33), times
 // `scale`, split into its even part e0 + cu^2 (e1 + e2 cu^2) and its odd part
@@ -165,8 +166,8 @@ struct PairCollision {
     for (int d = 0; d < D; ++d) {
       u[d] = j[d] * rr;
       // 1 / rho of a density below 1 rounds up more often than down: the quotient itself
-      // (the polynomial's error has room for it, see above)
-      if constexpr (!MA3) u[d] = fmaf(fmaf(-rho, u[d], j[d]), rr, u[d]);
+      // (not for FP16 populations, whose own rounding is a thousand times that)
+      if constexpr (!SC) u[d] = fmaf(fmaf(-rho, u[d], j[d]), rr, u[d]);
       asm("" : "+v"(u[d]));  // no longer a product: c.u adds them
     }
     if constexpr (FS == SRC_EDM)  // feq(rho, u + F / rho) - feq (ForcingScheme.h:184-197)
